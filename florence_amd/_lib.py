@@ -107,6 +107,8 @@ SIGNATURES = {
     "fl_mlp_adam": (ctypes.c_int, [_vp, _vp, _vp, _vp, ctypes.c_float, ctypes.c_float, ctypes.c_float,
                                    ctypes.c_float, _i32, _vp]),
     "fl_warmstart_features": (ctypes.c_int, [_vp, _vp, _vp, ctypes.c_double, _i64, _vp, _vp, _vp]),
+    "fl_warmstart_predict": (ctypes.c_int, [_vp, _vp, _vp, _vp, ctypes.c_double, _i64, _vp, _vp, _vp, _vp, _vp, _vp,
+                                            _vp, _vp]),
     "fl_warmstart_apply": (ctypes.c_int, [_vp, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp]),
 }
 

@@ -417,16 +417,13 @@ class WarmStartMLP(object):
         """out = prediction of the next converged displacement (Dirichlet dofs = ubc):
         the network's correction added to its base, the linear extrapolation
         2 u1 - u2, or ``base`` (the extrapolation of order base_order the network was
-        trained against; fl_warmstart_apply forms 2 a - b + correction, so a = b = base)."""
+        trained against; fl_warmstart_predict forms 2 a - b + correction, so a = b = base)."""
         lib = _lib.load()
-        nn = X.numel() // 3
-        b = self._buffers(nn)
-        self.features(X, u1, u2, lam, b["F"])
-        self.forward(b["F"], nn)
         a1, a2 = (u1, u2) if base is None else (base, base)
-        _lib.check(lib.fl_warmstart_apply(_lib.ptr(a1), _lib.ptr(a2), _lib.ptr(b["Y"]), nn, _lib.ptr(self.norm_out),
-                                          _lib.ptr(free_u8), _lib.ptr(ubc), _lib.ptr(out), _lib.stream_ptr()),
-                   "fl_warmstart_apply")
+        _lib.check(lib.fl_warmstart_predict(_lib.ptr(self.P), _lib.ptr(X), _lib.ptr(u1), _lib.ptr(u2), float(lam),
+                                            X.numel() // 3, _lib.ptr(self.norm_in), _lib.ptr(self.norm_out),
+                                            _lib.ptr(a1), _lib.ptr(a2), _lib.ptr(free_u8), _lib.ptr(ubc),
+                                            _lib.ptr(out), _lib.stream_ptr()), "fl_warmstart_predict")
         return out
 
     def train_step(self, F, T, n, lr, nout=3, ws=None, G=None, loss=None):

@@ -476,6 +476,9 @@ int fl_profile_read(int32_t *kinds, double *phase_ms, int32_t max_calls, int32_t
  *   with norm = device {mean[10], inv_std[10]}.
  * fl_warmstart_apply: u = free ? 2 u1 - u2 + out_norm[0..2] * Y + out_norm[3..5] : u_bc
  *   per dof (free_mask uint8 [3 nnode]).
+ * fl_warmstart_predict: the three in one launch -- the features of (X, u1, u2,
+ *   load_factor), the forward pass with parameters P, and
+ *   u = free ? 2 a - b + out_norm[0..2] * Y + out_norm[3..5] : u_bc.  Same values.
  */
 int64_t fl_mlp_param_count(void);
 size_t fl_mlp_workspace_size(int64_t n);
@@ -488,6 +491,10 @@ int fl_mlp_adam(float *P_dev, const float *Gr_dev, float *m_dev, float *v_dev, f
                 float eps, int32_t step, void *stream);
 int fl_warmstart_features(const double *X_dev, const double *u1_dev, const double *u2_dev, double load_factor,
                           int64_t nnode, const float *norm_dev, float *F_dev, void *stream);
+int fl_warmstart_predict(const float *P_dev, const double *X_dev, const double *u1_dev, const double *u2_dev,
+                         double load_factor, int64_t nnode, const float *norm_in_dev, const float *norm_out_dev,
+                         const double *a_dev, const double *b_dev, const uint8_t *free_mask_dev,
+                         const double *u_bc_dev, double *u_dev, void *stream);
 int fl_warmstart_apply(const double *u1_dev, const double *u2_dev, const float *Y_dev, int64_t nnode,
                        const float *out_norm_dev, const uint8_t *free_mask_dev, const double *u_bc_dev,
                        double *u_dev, void *stream);

@@ -180,3 +180,50 @@ def test_warmstart_feature_and_apply_kernels(cuda):
     corr = (on[:3].astype(np.float64) * Y[:, :3].astype(np.float64) + on[3:].astype(np.float64)).reshape(-1)
     refu = np.where(free == 1, 2 * u1.reshape(-1) - u2.reshape(-1) + corr, ubc)
     assert np.allclose(u.cpu().numpy(), refu, rtol=1e-14, atol=1e-14)
+
+
+@pytest.mark.parametrize("N", [1, 31, 33, 32 * 1024 + 7])
+def test_forward_row_remainders(cuda, N):
+    """Row counts that end inside a workgroup's 32 rows, and one past the grid's width
+    (some workgroups then run a second step on the weights they hold).  BF16 rounding
+    flips as above: 2e-3 norm-wise."""
+    P, X, T, dP, dX, dT = _setup(N, seed=N)
+    for got, ref in zip(_fwd(dP, dX), omlp.forward(P, X)):
+        assert _rel(got.cpu().numpy(), ref) < 2e-3
+
+
+@pytest.mark.parametrize("N,nout", [(32, 32), (32 * 257, 3)])
+def test_backward_partial_gradients(cuda, N, nout):
+    """One workgroup's gradient, and one row block more than there are workgroups."""
+    P, X, T, dP, dX, dT = _setup(N, nout, seed=N)
+    G, loss = _bwd(dP, dX, _fwd(dP, dX), dT, nout)
+    rloss, rg, _ = omlp.loss_and_grad(P, X, T, nout)
+    assert float(loss.item()) == pytest.approx(rloss, rel=1e-5)
+    gp, rp = omlp.unpack(G.cpu().numpy()), omlp.unpack(rg)
+    for name, _ in omlp.SHAPES:
+        assert _rel(gp[name], rp[name]) < 2e-3, name
+
+
+@pytest.mark.parametrize("nn", [1, 95, 32 * 1024 + 7])
+@pytest.mark.parametrize("based", [False, True])
+def test_predict_equals_its_three_parts(cuda, nn, based):
+    """fl_warmstart_predict against features, forward and apply: bit for bit."""
+    import torch
+    from florence_amd import _lib
+    from florence_amd.learned import WarmStartMLP
+    lib = _lib.load()
+    g = torch.Generator(device="cuda")
+    g.manual_seed(nn)
+    X, u1, u2, ubc, base = (torch.randn(3 * nn, generator=g, device="cuda", dtype=torch.float64) for _ in range(5))
+    free = (torch.rand(3 * nn, generator=g, device="cuda") < 0.8).to(torch.uint8)
+    net = WarmStartMLP(seed=2)
+    net.norm_in.copy_(torch.rand(20, generator=g, device="cuda"))
+    net.norm_out.copy_(torch.rand(6, generator=g, device="cuda"))
+    got = net.predict(X, u1, u2, 0.25, free, ubc, torch.empty_like(X), base if based else None)
+    F = torch.empty((nn, 32), dtype=torch.float32, device="cuda")
+    Y = net.forward(net.features(X, u1, u2, 0.25, F), nn)["Y"]
+    a, b = (base, base) if based else (u1, u2)
+    ref = torch.empty_like(X)
+    _lib.check(lib.fl_warmstart_apply(_lib.ptr(a), _lib.ptr(b), _lib.ptr(Y), nn, _lib.ptr(net.norm_out),
+                                      _lib.ptr(free), _lib.ptr(ubc), _lib.ptr(ref), _lib.stream_ptr()), "apply")
+    assert torch.equal(got, ref)
