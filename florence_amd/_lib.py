@@ -32,6 +32,7 @@ PRECISIONS = {"fp64": FL_PREC_FP64, "fp32": FL_PREC_FP32, "bf16": FL_PREC_BF16}
 FL_PREC_CSR32 = 16
 FL_TUNE_STIFF_SF = 7
 FL_TUNE_GATHER = 8
+FL_TUNE_CG = 9
 FL_RECORDS_D = 0
 FL_RECORDS_C = 1
 

@@ -4,6 +4,7 @@
 
 #include <cstdint>
 #include <cstdio>
+#include <mutex>
 #include <string>
 
 #include "../../include/florence_amd.h"
@@ -50,8 +51,12 @@ struct Carve {
 };
 
 // Kernel-variant knobs (set through fl_set_tuning; 0 = library default).
-enum TuneKey { TUNE_STIFF_MINW = 1, TUNE_STIFF_VARIANT_BASE = 2, TUNE_STIFF_SF = 7, TUNE_GATHER = 8, TUNE_KEYS = 9 };
+enum TuneKey { TUNE_STIFF_MINW = 1, TUNE_STIFF_VARIANT_BASE = 2, TUNE_STIFF_SF = 7, TUNE_GATHER = 8, TUNE_CG = 9, TUNE_KEYS = 10 };
 int tuning_value(int key, int dflt);
+
+// Held from the launch of a kernel whose workgroups wait for each other until it has ended:
+// two of them on one device could each hold part of the CUs and wait for the rest.
+std::mutex &persistent_lock(int device);
 
 // Order of the direct scatter table of hexes of p1^3 nodes: the order in which the
 // factorised stiffness kernel stores an element's entries.  Per element and slice az,

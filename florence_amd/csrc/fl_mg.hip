@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "fl_common.hpp"
+#include "fl_cg_persist.hpp"
 #include "fl_solve_kernels.hpp"
 
 namespace fl {
@@ -578,7 +579,10 @@ struct Mg {
     int coarse_its;
     LevelWork w[FL_MG_MAX_LEVELS];
     double *part;
-    double *s;   // [0, 8) FCG scalars, [8, 16) coarse CG scalars, [16] power-iteration norm
+    double *s;   // [0, 8) FCG scalars, [16] power-iteration norm, [20] coarse degrees, [24] bad block, [25] abort
+    CgpPlan cg;             // the coarsest level's CG in one launch (nw = 0: two launches per step)
+    uint64_t *slots;
+    int cg_runs;            // its launches so far: they alternate between two slot sets
     hipStream_t st;
 };
 
@@ -684,12 +688,34 @@ static int chebyshev(Mg &m, int l, const double *b, double **d_last) {
     return 0;
 }
 
-// fixed-step block-Jacobi CG from x = 0 on the coarsest level: x ~ A^-1 b (two
-// launches per step: cc_spmv_kernel, cc_update_kernel)
+// fixed-step block-Jacobi CG from x = 0 on the coarsest level: x ~ A^-1 b (one launch, or
+// two launches per step: cc_spmv_kernel, cc_update_kernel)
 static int coarse_solve(Mg &m, int l) {
     const FlMgLevel &L = m.lv[l];
     LevelWork &w = m.w[l];
     const int64_t nnode = L.nnode;
+    if (m.cg.nw) {
+        CgpArgs<double> a = {};
+        a.indptr = L.indptr;
+        a.nbr_ptr = L.node_nbr_ptr;
+        a.nbrs = L.node_nbrs;
+        a.V = lvals<double>(L);
+        a.nnode = nnode;
+        a.free_mask = L.free_mask;
+        a.P = w.P;
+        a.b = w.b;
+        a.x = w.x;
+        a.z[0] = w.d;
+        a.z[1] = w.d2;
+        a.slots = m.slots + (m.cg_runs & 1) * CGP_SLOTS;
+        a.slots_next = m.slots + (~m.cg_runs & 1) * CGP_SLOTS;
+        a.abort = reinterpret_cast<int32_t *>(m.s + 25);
+        a.maxit = m.coarse_its;
+        a.check_every = m.coarse_its + 1;
+        a.rtol = -1.0;
+        ++m.cg_runs;
+        return cgp_launch(m.cg, a, m.st);
+    }
     const int64_t ns = (nnode + CC_NB - 1) / CC_NB, nu = nb_v(nnode);
     double *z = w.d, *q = w.t2;
     double *pbuf[2] = {w.d2, w.t1};
@@ -784,7 +810,71 @@ static size_t carve_mg(Carve &cv, Mg &m, const FlMgLevel *lv, int nl) {
     }
     m.part = cv.take<double>((size_t)maxpart);
     m.s = cv.take<double>(32);
+    m.slots = cv.take<uint64_t>(2 * CGP_SLOTS);
     return cv.off + 256;
+}
+
+// The outer flexible CG on level 0.  *aborted: the coarsest level's one-launch CG gave up
+// waiting in some cycle, and x is no solution.
+static int fcg(Mg &m, const double *b, double *x, double *rO, double *rOld, double *p, double *q, double rtol,
+               int32_t maxit, int32_t check_every, int32_t *iterations, double *rel_residual, bool *aborted) {
+    const FlMgLevel *levels = m.lv;
+    const int64_t n0 = 3 * levels[0].nnode;
+    hipStream_t st = m.st;
+    double *s = m.s;
+    *aborted = false;
+    const unsigned nbv0 = nb_v(n0), nbs0 = nb_sp(levels[0].nnode);
+    fcg_start_kernel<<<nbv0, SV_T, 0, st>>>(n0, b, levels[0].free_mask, x, rO, m.part);
+    sum1_kernel<<<1, SV_T, 0, st>>>(m.part, nbv0, s + 4);
+    FL_LAUNCH_CHECK();
+    double bb = 0.0;
+    FL_HIP_CHECK(hipMemcpyAsync(&bb, s + 4, sizeof(double), hipMemcpyDeviceToHost, st));
+    FL_HIP_CHECK(hipStreamSynchronize(st));
+    const double bnorm = std::sqrt(bb);
+    *iterations = 0;
+    *rel_residual = 0.0;
+    if (bnorm == 0.0) return 0;
+    double *z = m.w[0].x;
+    int rc = vcycle(m, 0, rO);
+    if (rc) return rc;
+    fcg_dots_kernel<<<nbv0, SV_T, 0, st>>>(n0, z, rO, nullptr, m.part);
+    fcg_beta_kernel<<<1, SV_T, 0, st>>>(m.part, nbv0, s, 1);
+    fcg_dir_kernel<<<nbv0, SV_T, 0, st>>>(n0, s, z, p, 1);
+    FL_LAUNCH_CHECK();
+    double rel = 1.0;
+    int it = 0;
+    while (it < maxit) {
+        rc = level_spmv(m, 0, p, q, m.part);
+        if (rc) return rc;
+        const unsigned nch = (unsigned)((nbs0 + PART_CHUNK - 1) / PART_CHUNK);
+        part_sum_kernel<<<nch, SV_T, 0, st>>>(m.part, nbs0, m.part + nbs0);
+        fcg_alpha_kernel<<<1, SV_T, 0, st>>>(m.part + nbs0, nch, s);
+        fcg_update_kernel<<<nbv0, SV_T, 0, st>>>(n0, s, p, q, x, rO, rOld, m.part);
+        sum1_kernel<<<1, SV_T, 0, st>>>(m.part, nbv0, s + 4);
+        FL_LAUNCH_CHECK();
+        ++it;
+        if (it % check_every == 0 || it == maxit) {
+            double hs[22];   // s[4], and the abort flag in s[25]
+            FL_HIP_CHECK(hipMemcpyAsync(hs, s + 4, sizeof(hs), hipMemcpyDeviceToHost, st));
+            FL_HIP_CHECK(hipStreamSynchronize(st));
+            if (m.cg.nw && *reinterpret_cast<int32_t *>(hs + 21)) {
+                *aborted = true;
+                return 0;
+            }
+            rel = std::sqrt(hs[0]) / bnorm;
+            if (!(rel == rel) || rel <= rtol) break;
+        }
+        if (it == maxit) break;
+        rc = vcycle(m, 0, rO);
+        if (rc) return rc;
+        fcg_dots_kernel<<<nbv0, SV_T, 0, st>>>(n0, z, rO, rOld, m.part);
+        fcg_beta_kernel<<<1, SV_T, 0, st>>>(m.part, nbv0, s, 0);
+        fcg_dir_kernel<<<nbv0, SV_T, 0, st>>>(n0, s, z, p, 0);
+        FL_LAUNCH_CHECK();
+    }
+    *iterations = it;
+    *rel_residual = rel;
+    return 0;
 }
 
 }  // namespace
@@ -904,61 +994,31 @@ int fl_mg_pcg(const FlMgLevel *levels, int32_t nlevels, int32_t v32, const float
         const int rc = estimate_lmax(m, l, power_steps, power_warm != 0);
         if (rc) return rc;
     }
-    int32_t hbad = 0;
-    FL_HIP_CHECK(hipMemcpyAsync(&hbad, bad, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-    // outer flexible CG
-    const unsigned nbv0 = nb_v(n0), nbs0 = nb_sp(levels[0].nnode);
-    fcg_start_kernel<<<nbv0, SV_T, 0, st>>>(n0, b, levels[0].free_mask, x, rO, m.part);
-    sum1_kernel<<<1, SV_T, 0, st>>>(m.part, nbv0, s + 4);
+    int32_t hbad = 0, hdeg[3] = {0, 0, 0};
+    cgp_degree_kernel<<<(unsigned)((levels[nlevels - 1].nnode + 255) / 256), 256, 0, st>>>(
+        levels[nlevels - 1].node_nbr_ptr, levels[nlevels - 1].nnode, reinterpret_cast<int32_t *>(m.s + 20));
     FL_LAUNCH_CHECK();
-    double bb = 0.0;
-    FL_HIP_CHECK(hipMemcpyAsync(&bb, s + 4, sizeof(double), hipMemcpyDeviceToHost, st));
+    FL_HIP_CHECK(hipMemcpyAsync(&hbad, bad, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+    FL_HIP_CHECK(hipMemcpyAsync(&hdeg, m.s + 20, sizeof(hdeg), hipMemcpyDeviceToHost, st));
     FL_HIP_CHECK(hipStreamSynchronize(st));
     if (hbad) {
         set_error("fl_mg_pcg: singular diagonal block or missing diagonal entry");
         return FL_E_ARG;
     }
-    const double bnorm = std::sqrt(bb);
-    *iterations = 0;
-    *rel_residual = 0.0;
-    if (bnorm == 0.0) return 0;
-    double *z = m.w[0].x;
-    int rc = vcycle(m, 0, rO);
-    if (rc) return rc;
-    fcg_dots_kernel<<<nbv0, SV_T, 0, st>>>(n0, z, rO, nullptr, m.part);
-    fcg_beta_kernel<<<1, SV_T, 0, st>>>(m.part, nbv0, s, 1);
-    fcg_dir_kernel<<<nbv0, SV_T, 0, st>>>(n0, s, z, p, 1);
-    FL_LAUNCH_CHECK();
-    double rel = 1.0;
-    int it = 0;
-    while (it < maxit) {
-        rc = level_spmv(m, 0, p, q, m.part);
-        if (rc) return rc;
-        const unsigned nch = (unsigned)((nbs0 + PART_CHUNK - 1) / PART_CHUNK);
-        part_sum_kernel<<<nch, SV_T, 0, st>>>(m.part, nbs0, m.part + nbs0);
-        fcg_alpha_kernel<<<1, SV_T, 0, st>>>(m.part + nbs0, nch, s);
-        fcg_update_kernel<<<nbv0, SV_T, 0, st>>>(n0, s, p, q, x, rO, rOld, m.part);
-        sum1_kernel<<<1, SV_T, 0, st>>>(m.part, nbv0, s + 4);
-        FL_LAUNCH_CHECK();
-        ++it;
-        if (it % check_every == 0 || it == maxit) {
-            double rr = 0.0;
-            FL_HIP_CHECK(hipMemcpyAsync(&rr, s + 4, sizeof(double), hipMemcpyDeviceToHost, st));
-            FL_HIP_CHECK(hipStreamSynchronize(st));
-            rel = std::sqrt(rr) / bnorm;
-            if (!(rel == rel) || rel <= rtol) break;
-        }
-        if (it == maxit) break;
-        rc = vcycle(m, 0, rO);
-        if (rc) return rc;
-        fcg_dots_kernel<<<nbv0, SV_T, 0, st>>>(n0, z, rO, rOld, m.part);
-        fcg_beta_kernel<<<1, SV_T, 0, st>>>(m.part, nbv0, s, 0);
-        fcg_dir_kernel<<<nbv0, SV_T, 0, st>>>(n0, s, z, p, 0);
-        FL_LAUNCH_CHECK();
+    m.cg = cgp_plan(levels[nlevels - 1].nnode, hdeg[2], hdeg[0], (1 << 30) - hdeg[1]);
+    if (b == x) m.cg.nw = 0;   // the way back below reads b again
+    bool aborted = false;
+    if (m.cg.nw) {
+        int dev = 0;
+        FL_HIP_CHECK(hipGetDevice(&dev));
+        std::lock_guard<std::mutex> lock(persistent_lock(dev));
+        cgp_empty_kernel<<<(CGP_SLOTS + 255) / 256, 256, 0, st>>>(m.slots, CGP_SLOTS);
+        const int rc = fcg(m, b, x, rO, rOld, p, q, rtol, maxit, check_every, iterations, rel_residual, &aborted);
+        if (rc || !aborted) return rc;
+        // a workgroup of the coarse solve gave up waiting: again, step by step
+        m.cg.nw = 0;
     }
-    *iterations = it;
-    *rel_residual = rel;
-    return 0;
+    return fcg(m, b, x, rO, rOld, p, q, rtol, maxit, check_every, iterations, rel_residual, &aborted);
 }
 
 }  // extern "C"

@@ -12,9 +12,15 @@
 #include <vector>
 
 #include "fl_common.hpp"
+#include "fl_cg_persist.hpp"
 #include "fl_solve_kernels.hpp"
 
 namespace fl {
+
+std::mutex &persistent_lock(int device) {
+    static std::mutex m[64];
+    return m[device & 63];
+}
 
 template <typename VT>
 static int csr_spmv(const int32_t *indptr, const int32_t *node_nbr_ptr, const int32_t *node_nbrs, const VT *V,
@@ -52,28 +58,71 @@ static int pcg(const int32_t *indptr, const int32_t *node_nbr_ptr, const int32_t
     double *p = cv.take<double>(n);
     double *q = cv.take<double>(n);
     double *part = cv.take<double>(nb_sp + 2 * nb_v + 8);
-    double *s = cv.take<double>(8);
+    double *s = cv.take<double>(16);
     double *p2 = cv.take<double>(n);
+    uint64_t *slots = cv.take<uint64_t>(2 * CGP_SLOTS);
     if (!cv.ok) {
         set_error("%s: workspace too small (%zu < %zu)", name, workspace_bytes, cv.off);
         return FL_E_SPACE;
     }
     int32_t *bad = reinterpret_cast<int32_t *>(s + 7);
-    FL_HIP_CHECK(hipMemsetAsync(s, 0, sizeof(double) * 8, st));
+    FL_HIP_CHECK(hipMemsetAsync(s, 0, sizeof(double) * 16, st));
     block_jacobi_kernel<VT><<<(unsigned)((nnode + 255) / 256), 256, 0, st>>>(indptr, node_nbr_ptr, node_nbrs, V, nnode,
                                                                         free_mask, P, bad);
+    cgp_degree_kernel<<<(unsigned)((nnode + 255) / 256), 256, 0, st>>>(node_nbr_ptr, nnode,
+                                                                       reinterpret_cast<int32_t *>(s + 8));
     FL_LAUNCH_CHECK();
-    cg_start_kernel<<<(unsigned)nb_v, SV_T, 0, st>>>(nnode, P, b, free_mask, x, r, z, p, part);
-    FL_LAUNCH_CHECK();
-    reduce2_kernel<<<1, SV_T, 0, st>>>(part, nb_v, s + 0, s + 6);   // rz, bb (= r0.r0)
-    FL_LAUNCH_CHECK();
-    double hs[8];
+    double hs[16];
     FL_HIP_CHECK(hipMemcpyAsync(hs, s, sizeof(hs), hipMemcpyDeviceToHost, st));
     FL_HIP_CHECK(hipStreamSynchronize(st));
     if (*reinterpret_cast<int32_t *>(&hs[7])) {
         set_error("%s: singular diagonal block or missing diagonal entry", name);
         return FL_E_ARG;
     }
+    const int32_t *deg = reinterpret_cast<const int32_t *>(hs + 8);
+    const CgpPlan plan = cgp_plan(nnode, deg[2], deg[0], (1 << 30) - deg[1]);
+    if (plan.nw) {
+        // the whole solve in one launch
+        CgpArgs<VT> a = {};
+        a.indptr = indptr;
+        a.nbr_ptr = node_nbr_ptr;
+        a.nbrs = node_nbrs;
+        a.V = V;
+        a.nnode = nnode;
+        a.free_mask = free_mask;
+        a.P = P;
+        a.b = b;
+        a.x = x;
+        a.z[0] = z;
+        a.z[1] = p;
+        a.slots = slots;
+        a.slots_next = slots + CGP_SLOTS;
+        a.abort = reinterpret_cast<int32_t *>(s + 12);
+        a.out = s + 13;
+        a.maxit = maxit;
+        a.check_every = check_every;
+        a.rtol = rtol;
+        int dev = 0;
+        FL_HIP_CHECK(hipGetDevice(&dev));
+        std::lock_guard<std::mutex> lock(persistent_lock(dev));
+        cgp_empty_kernel<<<(CGP_SLOTS + 255) / 256, 256, 0, st>>>(slots, CGP_SLOTS);
+        const int rc = cgp_launch(plan, a, st);
+        if (rc) return rc;
+        FL_HIP_CHECK(hipMemcpyAsync(hs, s, sizeof(hs), hipMemcpyDeviceToHost, st));
+        FL_HIP_CHECK(hipStreamSynchronize(st));
+        if (!*reinterpret_cast<int32_t *>(&hs[12])) {
+            *iterations = (int32_t)hs[13];
+            *rel_residual = hs[14];
+            return 0;
+        }
+        // a workgroup gave up waiting (the device was not this process's alone): step by step
+    }
+    cg_start_kernel<<<(unsigned)nb_v, SV_T, 0, st>>>(nnode, P, b, free_mask, x, r, z, p, part);
+    FL_LAUNCH_CHECK();
+    reduce2_kernel<<<1, SV_T, 0, st>>>(part, nb_v, s + 0, s + 6);   // rz, bb (= r0.r0)
+    FL_LAUNCH_CHECK();
+    FL_HIP_CHECK(hipMemcpyAsync(hs, s, sizeof(hs), hipMemcpyDeviceToHost, st));
+    FL_HIP_CHECK(hipStreamSynchronize(st));
     const double bnorm = std::sqrt(hs[6]);
     *iterations = 0;
     *rel_residual = 0.0;
@@ -116,7 +165,8 @@ size_t fl_pcg_workspace_size(int64_t nnode) {
     const int64_t n = 3 * nnode;
     const int64_t nb_sp = (nnode + SP_W - 1) / SP_W, nb_v = (nnode + SV_T - 1) / SV_T;
     return align_up(sizeof(double) * 9 * nnode, 256) + 5 * align_up(sizeof(double) * n, 256) +
-           align_up(sizeof(double) * (nb_sp + 2 * nb_v + 8), 256) + align_up(sizeof(double) * 8, 256) + 1024;
+           align_up(sizeof(double) * (nb_sp + 2 * nb_v + 8), 256) + align_up(sizeof(double) * 16, 256) +
+           align_up(sizeof(uint64_t) * 2 * CGP_SLOTS, 256) + 1024;
 }
 
 int fl_csr_spmv(const int32_t *indptr, const int32_t *node_nbr_ptr, const int32_t *node_nbrs, const double *V,

@@ -456,6 +456,11 @@ int32_t fl_stiffness_variant_count(int32_t np_class);
  * time instead of loading eight elements' rows first; bit 1: nodes inside one element
  * go through the general kernel instead of the single-element one.  Same V and T. */
 #define FL_TUNE_GATHER 8
+/* key 9: block-Jacobi CG (fl_pcg, fl_mg_pcg's coarsest level) -- 1: one launch per step's
+ * part for every matrix; 2: the one-launch form gives up its first wait, and the solve
+ * falls back to the other (the results are those of 1).  Default: one launch per solve
+ * where the matrix fits the chip's registers. */
+#define FL_TUNE_CG 9
 int fl_set_tuning(int32_t key, int32_t value);
 int fl_profile_read(int32_t *kinds, double *phase_ms, int32_t max_calls, int32_t max_phases);
 

@@ -350,3 +350,29 @@ def spmv_masked(ln, x, live):
     y = torch.empty_like(x)
     spmv(ln.dm, ln.V, x, y, mask)
     return y * mask.to(y.dtype)
+
+
+def test_coarse_cg_in_one_launch(cuda):
+    """The coarsest level's CG as one launch: the solve agrees with the launch-per-step form
+    (both to 1e-12 on the residual: 1e-9 on the solution), repeats bitwise, and a coarse
+    solve that gives up its first wait restarts in the launch-per-step form, bitwise."""
+    import torch
+    from florence_amd import _lib
+    from florence_amd.assembly import DeviceMeshData, assemble_device
+    from florence_amd.multigrid import MultigridSolver
+    m, fs, mat = cube_hex_p4(3)
+    dm = DeviceMeshData(m, fs)
+    V, _, _ = assemble_device(dm, mat, twisted_state(m, 5.0))
+    free = torch.as_tensor(np.isnan(clamp_and_twist(m)).ravel().astype(np.uint8), device=cuda)
+    b = torch.as_tensor(np.random.default_rng(0).standard_normal(free.numel()), device=cuda) * free
+    lib = _lib.load()
+    x = {}
+    try:
+        for mode in (0, 1, 2):
+            _lib.check(lib.fl_set_tuning(_lib.FL_TUNE_CG, mode), "fl_set_tuning")
+            x[mode] = [MultigridSolver(rtol=1e-12).Solve(dm, V, free, b, torch.empty_like(b)) for _ in range(2)]
+            assert torch.equal(x[mode][0], x[mode][1])
+    finally:
+        lib.fl_set_tuning(_lib.FL_TUNE_CG, 0)
+    assert torch.equal(x[1][0], x[2][0])
+    assert float(torch.linalg.norm(x[0][0] - x[1][0]) / torch.linalg.norm(x[1][0])) <= 1e-9

@@ -64,3 +64,59 @@ def test_pcg_solves_reduced_system(cuda):
     print("pcg iterations", ls.iterations, "rel err", err, flush=True)
     assert err < 1e-9
     assert np.all(x.cpu().numpy()[free == 0] == 0.0)
+
+
+# 3x3 blocks per matrix: one workgroup; a few threads' worth each; two, four and six blocks per
+# thread on the whole chip; above the one-launch form's reach
+@pytest.mark.parametrize("element,p,n,csr", [("tet", 1, 1, "fp64"), ("hex", 1, 2, "fp64"), ("tet", 2, 4, "fp32"),
+                                             ("tet", 2, 8, "fp64"), ("tet", 1, 17, "fp64"), ("hex", 1, 18, "fp32"),
+                                             ("hex", 2, 8, "fp64"), ("hex", 2, 9, "fp64"), ("hex", 3, 9, "fp64")])
+def test_pcg_in_one_launch(cuda, element, p, n, csr):
+    """The one-launch CG against the launch-per-step one on the same system: both reach
+    1e-10 (the true residual, by a product with the CSR, within the recursion's drift of
+    it), a second solve is bitwise equal, and a solve whose first wait is given up equals
+    the launch-per-step one bitwise."""
+    import torch
+    from cases import cube_mesh, function_space
+    from florence_amd import _lib
+    from florence_amd.assembly import DeviceMeshData, assemble_device
+    from florence_amd.materials import NeoHookean
+    from florence_amd.solver import LinearSolver, spmv
+    m = cube_mesh(element, p, n, jitter=0.02, seed=n)
+    dm = DeviceMeshData(m, function_space(m, p))
+    V, _, _ = assemble_device(dm, NeoHookean(3, mu=1.0, lamb=10.0), m.points, precision=csr, csr=csr)
+    free = np.isnan(clamp_and_pull(m).ravel()).astype(np.uint8)
+    f = torch.as_tensor(free, device=cuda)
+    b = torch.as_tensor(np.random.default_rng(n).standard_normal(free.size) * free, device=cuda)
+    lib = _lib.load()
+    x, its = {}, {}
+    try:
+        for mode in (0, 1, 2):
+            _lib.check(lib.fl_set_tuning(_lib.FL_TUNE_CG, mode), "fl_set_tuning")
+            ls = LinearSolver(rtol=1e-10, check_every=1)
+            x[mode] = ls.Solve(dm, V, f, b, torch.full_like(b, float("nan"))).clone()
+            again = ls.Solve(dm, V, f, b, torch.empty_like(b))
+            assert torch.equal(x[mode], again)
+            its[mode] = ls.iterations[0]
+    finally:
+        lib.fl_set_tuning(_lib.FL_TUNE_CG, 0)
+    assert torch.equal(x[1], x[2]) and its[1] == its[2]
+    y = torch.empty_like(b)
+    for mode in (0, 1):
+        spmv(dm, V, x[mode], y, f)
+        rel = float(torch.linalg.norm((b - y) * f) / torch.linalg.norm(b))
+        print(element, p, n, csr, "mode", mode, its[mode], "iterations, residual", rel)
+        assert rel <= 1.1e-10
+        assert torch.all(x[mode][f == 0] == 0)
+    assert abs(its[0] - its[1]) <= max(2, its[1] // 20)
+
+
+def test_pcg_zero_right_hand_side(cuda):
+    import torch
+    from florence_amd.solver import LinearSolver
+    m, dm, V, K = _setup()
+    free = torch.as_tensor(np.isnan(clamp_and_pull(m).ravel()).astype(np.uint8), device=cuda)
+    ls = LinearSolver()
+    x = ls.Solve(dm, V, free, torch.zeros(K.shape[0], dtype=torch.float64, device=cuda),
+                 torch.full((K.shape[0],), 3.0, dtype=torch.float64, device=cuda))
+    assert ls.iterations == [0] and torch.all(x == 0)
