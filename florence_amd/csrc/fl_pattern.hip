@@ -120,24 +120,55 @@ __global__ void fill_incidence_kernel(const int32_t *__restrict__ elements, int6
     node_elem[offsets[nd] + slot] = (int32_t)t;   // t = e*npe + local
 }
 
-// Sort each node's incidence list (ascending element, hence ascending e*npe+local)
-// and emit the int32 pointer array.  Lists are short (<= a few dozen entries).
-__global__ void sort_incidence_kernel(const int64_t *__restrict__ offsets, int64_t nnode,
-                                      int32_t *__restrict__ node_elem, int32_t *__restrict__ node_elem_ptr) {
-    const int64_t a = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// Sort each node's incidence list (ascending element, hence ascending e*npe+local) and emit
+// the int32 pointer array: sixteen lanes per node hold the list in registers, and an
+// entry's place is the number of smaller ones (in place: a list's reads precede its
+// writes in the same wave).  Lists of more than 64 entries: insertion by one lane, the
+// only form before, which walked every list through memory (61 us on 24k tet p=2 nodes).
+constexpr int SI_L = 16, SI_N = 64;
+__global__ __launch_bounds__(256) void sort_incidence_kernel(const int64_t *__restrict__ offsets, int64_t nnode,
+                                                             int32_t *__restrict__ node_elem,
+                                                             int32_t *__restrict__ node_elem_ptr) {
+    const int64_t a = ((int64_t)blockIdx.x * 256 + threadIdx.x) / SI_L;
+    const int gl = threadIdx.x % SI_L;
     if (a > nnode) return;
-    node_elem_ptr[a] = (int32_t)offsets[a];
+    if (gl == 0) node_elem_ptr[a] = (int32_t)offsets[a];
     if (a == nnode) return;
-    const int64_t b = offsets[a], e = offsets[a + 1];
-    for (int64_t i = b + 1; i < e; ++i) {
-        const int32_t v = node_elem[i];
-        int64_t j = i - 1;
-        while (j >= b && node_elem[j] > v) {
-            node_elem[j + 1] = node_elem[j];
-            --j;
+    const int64_t b = offsets[a];
+    const int n = (int)(offsets[a + 1] - b);
+    int32_t *list = node_elem + b;
+    if (n > SI_N) {
+        if (gl != 0) return;
+        for (int i = 1; i < n; ++i) {
+            const int32_t v = list[i];
+            int j = i - 1;
+            while (j >= 0 && list[j] > v) {
+                list[j + 1] = list[j];
+                --j;
+            }
+            list[j + 1] = v;
         }
-        node_elem[j + 1] = v;
+        return;
     }
+    constexpr int U = SI_N / SI_L;
+    int32_t v[U];
+    int rank[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        v[u] = gl + SI_L * u < n ? list[gl + SI_L * u] : INT_MAX;
+        rank[u] = 0;
+    }
+#pragma unroll
+    for (int w = 0; w < U; ++w)
+        if (SI_L * w < n)
+            for (int j = 0; j < SI_L; ++j) {
+                const int32_t x = __shfl(v[w], j, SI_L);
+#pragma unroll
+                for (int u = 0; u < U; ++u) rank[u] += x < v[u];
+            }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (gl + SI_L * u < n) list[rank[u]] = v[u];
 }
 
 // ----------------------------------------------------------- neighbour lists
@@ -201,66 +232,159 @@ __device__ int gather_sort_unique(const int32_t *__restrict__ elements, int32_t 
     return flag_sum[NB_T - 1];
 }
 
-__global__ __launch_bounds__(NB_T) void count_neighbours_kernel(
+// Nodes of at most NW_MAX candidates: one wave per node, its candidates sorted in the
+// wave's own 4 KB of LDS without a workgroup barrier (a wave's LDS accesses are in order;
+// the fences only keep the compiler's).  The workgroup form below, for the nodes above
+// that, sorted every list before: its 33 KB of LDS and two dozen barriers for lists of
+// mostly under 64 candidates took 292 + 170 us on 24k tet p=2 nodes; this form
+// takes 28 + 33.
+constexpr int NW_MAX = 1024;
+
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// the rows of node a (cnt neighbours in c, list start p0): indptr, and every row's columns
+__device__ __forceinline__ void write_rows(const int32_t *c, int cnt, int64_t a, int64_t nnode, int32_t p0,
+                                           const int32_t *__restrict__ node_nbr_ptr, int32_t *__restrict__ indptr,
+                                           int32_t *__restrict__ indices, int t, int nt) {
+    const int rowlen = 3 * cnt;
+    if (t < 3) indptr[3 * a + t] = (int32_t)(9 * (int64_t)p0 + t * rowlen);
+    // the last entry holds a negative flag as well (fl_pattern_fill): added, not stored
+    if (a == nnode - 1 && t == 0) atomicAdd(indptr + 3 * nnode, (int32_t)(9 * (int64_t)node_nbr_ptr[nnode]));
+    if (indices == nullptr) return;
+    for (int q = t; q < 3 * rowlen; q += nt) {
+        const int i = q >= 2 * rowlen ? 2 : (q >= rowlen ? 1 : 0);
+        const int col = q - i * rowlen, r = col / 3;
+        indices[9 * (int64_t)p0 + q] = 3 * c[r] + (col - 3 * r);
+    }
+}
+
+constexpr int32_t FILL_BAD = INT32_MIN;   // in indptr[3 nnode]: lists inconsistent with the counts
+
+template <bool FILL>
+__global__ __launch_bounds__(256) void wave_neighbours_kernel(
     const int32_t *__restrict__ elements, int32_t npe, const int32_t *__restrict__ node_elem_ptr,
     const int32_t *__restrict__ node_elem, int64_t nnode, int64_t *__restrict__ nbr_count,
-    int32_t *__restrict__ max_degree, int32_t *__restrict__ overflow) {
-    __shared__ int32_t cand[NB_MAX];
-    __shared__ int32_t flag_sum[NB_T];
-    const int64_t a = blockIdx.x;
-    const int cnt = gather_sort_unique(elements, npe, node_elem_ptr, node_elem, a, cand, flag_sum, overflow);
-    if (threadIdx.x == 0) {
-        nbr_count[a] = cnt < 0 ? 0 : cnt;
-        if (cnt > 0) atomicMax(max_degree, cnt);
-    }
-}
-
-__global__ __launch_bounds__(NB_T) void fill_neighbours_kernel(
-    const int32_t *__restrict__ elements, int32_t npe, const int32_t *__restrict__ node_elem_ptr,
-    const int32_t *__restrict__ node_elem, int64_t nnode, const int32_t *__restrict__ node_nbr_ptr,
-    int32_t *__restrict__ node_nbrs, int32_t *__restrict__ indptr, int32_t *__restrict__ indices,
-    int32_t *__restrict__ overflow) {
-    __shared__ int32_t cand[NB_MAX];
-    __shared__ int32_t flag_sum[NB_T];
-    const int64_t a = blockIdx.x;
-    const int t = threadIdx.x;
-    const int cnt = gather_sort_unique(elements, npe, node_elem_ptr, node_elem, a, cand, flag_sum, overflow);
-    if (cnt < 0) return;
-    const int32_t p0 = node_nbr_ptr[a];
-    if (cnt != node_nbr_ptr[a + 1] - p0) {
-        if (t == 0) atomicOr(overflow, 2);
-        return;
-    }
-    const int32_t b0 = node_elem_ptr[a], b1 = node_elem_ptr[a + 1];
-    const int ncand = (b1 - b0) * npe;
+    const int32_t *__restrict__ node_nbr_ptr, int32_t *__restrict__ node_nbrs, int32_t *__restrict__ indptr,
+    int32_t *__restrict__ indices) {
+    __shared__ int32_t sc[4][NW_MAX];
+    const int lane = threadIdx.x & 63;
+    int32_t *c = sc[threadIdx.x >> 6];
+    const int64_t a = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (a >= nnode) return;
+    const int32_t b0 = node_elem_ptr[a];
+    const int64_t nc = (int64_t)(node_elem_ptr[a + 1] - b0) * npe;
+    if (nc > NW_MAX) return;
+    const int ncand = (int)nc;
     int S = 64;
     while (S < ncand) S <<= 1;
-    const int per = (S + NB_T - 1) / NB_T;
-    const int lo = t * per, hi = min(lo + per, ncand);
-    int r = t == 0 ? 0 : flag_sum[t - 1];
-    for (int i = lo; i < hi; ++i) {
-        if (i == 0 || cand[i] != cand[i - 1]) {
-            node_nbrs[p0 + r] = cand[i];
-            ++r;
+    for (int i = lane; i < S; i += 64) {
+        int32_t v = INT_MAX;
+        if (i < ncand) {
+            const int j = i / npe;
+            const uint32_t e = (uint32_t)node_elem[b0 + j] / (uint32_t)npe;
+            v = elements[(int64_t)e * npe + (i - j * npe)];
         }
+        c[i] = v;
     }
-    __syncthreads();
-    // CSR rows 3a+i: indptr = 9*p0 + i*3*cnt; columns 3b+k
-    const int64_t rowlen = 3 * (int64_t)cnt;
-    if (t < 3) indptr[3 * a + t] = (int32_t)(9 * (int64_t)p0 + t * rowlen);
-    if (a == nnode - 1 && t == 0) indptr[3 * nnode] = (int32_t)(9 * (int64_t)node_nbr_ptr[nnode]);
-    if (indices != nullptr) {
-        for (int64_t q = t; q < 3 * rowlen; q += NB_T) {
-            const int64_t i = q / rowlen, c = q % rowlen;
-            const int32_t nb = node_nbrs[p0 + c / 3];
-            indices[9 * (int64_t)p0 + i * rowlen + c] = 3 * nb + (int32_t)(c % 3);
+    wave_fence();
+    for (int k = 2; k <= S; k <<= 1)
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            for (int t = lane; t < S / 2; t += 64) {
+                const int i = ((t & ~(j - 1)) << 1) | (t & (j - 1)), p = i | j;
+                const int32_t x = c[i], y = c[p];
+                if ((x > y) == ((i & k) == 0)) {
+                    c[i] = y;
+                    c[p] = x;
+                }
+            }
+            wave_fence();
         }
+    // the distinct ones, packed to the front (an entry only moves down, past entries read)
+    int cnt = 0;
+    for (int i0 = 0; i0 < ncand; i0 += 64) {
+        const int i = i0 + lane;
+        const int32_t v = i < ncand ? c[i] : 0;
+        const bool first = i < ncand && (i == 0 || c[i - 1] != v);
+        wave_fence();
+        const unsigned long long m = __ballot(first);
+        if (first) c[cnt + __popcll(m & ((1ull << lane) - 1))] = v;
+        cnt += __popcll(m);
+        wave_fence();
+    }
+    if constexpr (!FILL) {
+        if (lane == 0) nbr_count[a] = cnt;
+    } else {
+        const int32_t p0 = node_nbr_ptr[a];
+        if (cnt != node_nbr_ptr[a + 1] - p0) {
+            if (lane == 0) atomicOr(indptr + 3 * nnode, FILL_BAD);
+            return;
+        }
+        for (int i = lane; i < cnt; i += 64) node_nbrs[p0 + i] = c[i];
+        write_rows(c, cnt, a, nnode, p0, node_nbr_ptr, indptr, indices, lane, 64);
     }
 }
 
-__global__ void i64_to_i32_kernel(const int64_t *__restrict__ src, int32_t *__restrict__ dst, int64_t n) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) dst[t] = (int32_t)src[t];
+// The nodes of more than NW_MAX candidates, one workgroup per node: a grid of fixed size
+// looks through the nodes 256 at a time and takes up the large ones.
+template <bool FILL>
+__global__ __launch_bounds__(NB_T) void group_neighbours_kernel(
+    const int32_t *__restrict__ elements, int32_t npe, const int32_t *__restrict__ node_elem_ptr,
+    const int32_t *__restrict__ node_elem, int64_t nnode, int64_t *__restrict__ nbr_count,
+    int32_t *__restrict__ overflow, const int32_t *__restrict__ node_nbr_ptr,
+    int32_t *__restrict__ node_nbrs, int32_t *__restrict__ indptr, int32_t *__restrict__ indices) {
+    __shared__ int32_t cand[NB_MAX];
+    __shared__ int32_t flag_sum[NB_T];
+    __shared__ unsigned long long large[NB_T / 64];
+    const int t = threadIdx.x;
+    for (int64_t base = (int64_t)blockIdx.x * NB_T; base < nnode; base += (int64_t)gridDim.x * NB_T) {
+        const bool mine = base + t < nnode &&
+                          (int64_t)(node_elem_ptr[base + t + 1] - node_elem_ptr[base + t]) * npe > NW_MAX;
+        const unsigned long long m = __ballot(mine);
+        if ((t & 63) == 0) large[t >> 6] = m;
+        __syncthreads();
+        for (int w = 0; w < NB_T / 64; ++w)
+            for (unsigned long long rest = large[w]; rest; rest &= rest - 1) {
+                const int64_t a = base + 64 * w + __ffsll((long long)rest) - 1;
+                __syncthreads();   // the previous node's last reads of cand and flag_sum
+                const int cnt = gather_sort_unique(elements, npe, node_elem_ptr, node_elem, a, cand, flag_sum,
+                                                   overflow);
+                if constexpr (!FILL) {
+                    if (t == 0) nbr_count[a] = cnt < 0 ? 0 : cnt;
+                } else {
+                    const int32_t p0 = node_nbr_ptr[a];
+                    if (cnt < 0 || cnt != node_nbr_ptr[a + 1] - p0) {
+                        if (t == 0) atomicOr(indptr + 3 * nnode, FILL_BAD);
+                        continue;
+                    }
+                    const int ncand = (node_elem_ptr[a + 1] - node_elem_ptr[a]) * npe;
+                    int S = 64;
+                    while (S < ncand) S <<= 1;
+                    const int per = (S + NB_T - 1) / NB_T;
+                    const int lo = t * per, hi = min(lo + per, ncand);
+                    int r = t == 0 ? 0 : flag_sum[t - 1];
+                    for (int i = lo; i < hi; ++i)
+                        if (i == 0 || cand[i] != cand[i - 1]) node_nbrs[p0 + r++] = cand[i];
+                    __syncthreads();
+                    write_rows(node_nbrs + p0, cnt, a, nnode, p0, node_nbr_ptr, indptr, indices, t, NB_T);
+                }
+            }
+        __syncthreads();   // before the next nodes' masks
+    }
+}
+
+// node_nbr_ptr from the scanned counts, and the largest count (one atomic per wave that
+// has a larger one than is recorded)
+__global__ __launch_bounds__(256) void nbr_ptr_kernel(const int64_t *__restrict__ src, int32_t *__restrict__ dst,
+                                                      int64_t nnode, int32_t *__restrict__ max_degree) {
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (t <= nnode) dst[t] = (int32_t)src[t];
+    int d = t < nnode ? (int)(src[t + 1] - src[t]) : 0;
+    for (int off = 32; off > 0; off >>= 1) d = max(d, __shfl_xor(d, off, 64));
+    if ((threadIdx.x & 63) == 0 && d > __hip_atomic_load(max_degree, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(max_degree, d);
 }
 
 // ranks[(e npe + la) npe + lb] = position of node elements[e][lb] in the sorted
@@ -343,6 +467,104 @@ __global__ void scatter_table_kernel(const int32_t *__restrict__ elements, int64
     table[t] = ok ? (int16_t)(add ? lo - 32768 : lo) : (int16_t)0;
 }
 
+static unsigned group_grid(int64_t nnode) { return (unsigned)std::min<int64_t>((nnode + NB_T - 1) / NB_T, 1024); }
+
+// ------------------------------------------------------------------- gather plan
+// Node classes by neighbour count: class 0 the smallest count (in meshes with
+// element-interior nodes, exactly those: a node of two distinct elements has more
+// neighbours than an element has nodes), classes 1.. by at most 128, 256, ... 2048.  The
+// nodes are grouped by class in ascending order: counts per chunk of PL_CHUNK nodes,
+// their scan per class, and a stable scatter.
+constexpr int PL_CHUNK = 1024, PL_C = FL_GATHER_BUCKETS;
+// scratch (int32, zeroed): [0] 2^30 - smallest count, [1, 7) largest count per class, [7, 13)
+// nodes per class, [13] largest count above every class; from 16: [chunk][class]
+constexpr int PL_HEAD = 16;
+__device__ __forceinline__ int plan_class(int d, int dmin) {
+    if (d == dmin) return 0;
+    int c = 1;
+    while (c < PL_C && d > (64 << c)) ++c;
+    return c;
+}
+
+__global__ __launch_bounds__(256) void plan_min_kernel(const int32_t *__restrict__ ptr, int64_t nnode,
+                                                       int32_t *__restrict__ w) {
+    const int64_t a = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    int m = a < nnode ? (1 << 30) - (ptr[a + 1] - ptr[a]) : 0;
+    for (int off = 32; off > 0; off >>= 1) m = max(m, __shfl_xor(m, off, 64));
+    if ((threadIdx.x & 63) == 0 && m > __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(w, m);
+}
+
+// SCATTER = false: counts and largest degrees of a chunk's classes; true: its nodes put in
+// their places (the chunk counts scanned before)
+template <bool SCATTER>
+__global__ __launch_bounds__(256) void plan_chunk_kernel(const int32_t *__restrict__ ptr, int64_t nnode,
+                                                         int32_t *__restrict__ w, int32_t *__restrict__ order) {
+    __shared__ int32_t cnt[4][PL_C], base[PL_C], deg[PL_C + 1];
+    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+    const int dmin = (1 << 30) - w[0];
+    int32_t *hist = w + PL_HEAD + PL_C * (int64_t)blockIdx.x;
+    if (t < PL_C) base[t] = SCATTER ? hist[t] : 0;
+    if (t < PL_C + 1) deg[t] = 0;
+    __syncthreads();
+    for (int r = 0; r < PL_CHUNK / 256; ++r) {
+        const int64_t a = (int64_t)blockIdx.x * PL_CHUNK + 256 * r + t;
+        const int d = a < nnode ? ptr[a + 1] - ptr[a] : 0;
+        const int c = a < nnode ? plan_class(d, dmin) : -1;
+        if (!SCATTER && c >= 0 && d > deg[c]) atomicMax(&deg[c], d);
+        int before = 0;
+#pragma unroll
+        for (int k = 0; k < PL_C; ++k) {
+            const unsigned long long m = __ballot(c == k);
+            if (c == k) before = __popcll(m & ((1ull << lane) - 1));
+            if (lane == 0) cnt[wave][k] = __popcll(m);
+        }
+        __syncthreads();
+        if (SCATTER && c >= 0 && c < PL_C) {
+            for (int v = 0; v < wave; ++v) before += cnt[v][c];
+            order[base[c] + before] = (int32_t)a;
+        }
+        __syncthreads();
+        if (t < PL_C) base[t] += cnt[0][t] + cnt[1][t] + cnt[2][t] + cnt[3][t];
+        __syncthreads();
+    }
+    if (!SCATTER) {
+        if (t < PL_C) {
+            hist[t] = base[t];
+            if (deg[t]) atomicMax(w + 1 + t, deg[t]);
+        }
+        if (t == PL_C && deg[t]) atomicMax(w + 13, deg[t]);
+    }
+}
+
+// chunk counts -> first places, one wave per class; then the class's own start is added
+__global__ __launch_bounds__(64 * PL_C) void plan_scan_kernel(int32_t *__restrict__ w, int64_t nchunk) {
+    __shared__ int32_t total[PL_C];
+    const int c = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    int32_t *h = w + PL_HEAD + c;
+    int s = 0;
+    for (int64_t b = lane; b < nchunk; b += 64) s += h[PL_C * b];
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if (lane == 0) {
+        total[c] = s;
+        w[7 + c] = s;
+    }
+    __syncthreads();
+    int run = 0;
+    for (int k = 0; k < c; ++k) run += total[k];
+    for (int64_t b0 = 0; b0 < nchunk; b0 += 64) {
+        const int64_t b = b0 + lane;
+        const int v = b < nchunk ? h[PL_C * b] : 0;
+        int x = v;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int y = __shfl_up(x, off, 64);
+            if (lane >= off) x += y;
+        }
+        if (b < nchunk) h[PL_C * b] = run + x - v;
+        run += __shfl(x, 63, 64);
+    }
+}
+
 }  // namespace fl
 
 using namespace fl;
@@ -394,15 +616,20 @@ int fl_pattern_graph(const int32_t *elements, int64_t nelem, int32_t npe, int64_
     if (rc) return rc;
     fill_incidence_kernel<<<gb, 256, 0, st>>>(elements, nent, counts, cursor, node_elem);
     FL_LAUNCH_CHECK();
-    sort_incidence_kernel<<<(unsigned)((nnode + 1 + 255) / 256), 256, 0, st>>>(counts, nnode, node_elem,
-                                                                               node_elem_ptr);
+    sort_incidence_kernel<<<(unsigned)(((nnode + 1) * SI_L + 255) / 256), 256, 0, st>>>(counts, nnode, node_elem,
+                                                                                        node_elem_ptr);
     FL_LAUNCH_CHECK();
     FL_HIP_CHECK(hipMemsetAsync(nbrc, 0, sizeof(int64_t) * (nnode + 1), st));
-    count_neighbours_kernel<<<(unsigned)nnode, NB_T, 0, st>>>(elements, npe, node_elem_ptr, node_elem, nnode, nbrc,
-                                                              flags + 2, flags + 1);
+    wave_neighbours_kernel<false><<<(unsigned)((nnode + 3) / 4), 256, 0, st>>>(
+        elements, npe, node_elem_ptr, node_elem, nnode, nbrc, nullptr, nullptr, nullptr, nullptr);
+    group_neighbours_kernel<false><<<group_grid(nnode), NB_T, 0, st>>>(elements, npe, node_elem_ptr, node_elem, nnode,
+                                                                      nbrc, flags + 1, nullptr, nullptr,
+                                                                      nullptr, nullptr);
     FL_LAUNCH_CHECK();
     rc = exclusive_scan_i64(nbrc, nnode + 1, scratch, sc, st);
     if (rc) return rc;
+    nbr_ptr_kernel<<<(unsigned)((nnode + 1 + 255) / 256), 256, 0, st>>>(nbrc, node_nbr_ptr, nnode, flags + 2);
+    FL_LAUNCH_CHECK();
     int64_t total = 0;
     int32_t hflags[4] = {0, 0, 0, 0};
     FL_HIP_CHECK(hipMemcpyAsync(&total, nbrc + nnode, sizeof(int64_t), hipMemcpyDeviceToHost, st));
@@ -420,9 +647,6 @@ int fl_pattern_graph(const int32_t *elements, int64_t nelem, int32_t npe, int64_
         set_error("fl_pattern_graph: nnz = %lld exceeds int32 CSR indices", (long long)(9 * total));
         return FL_E_LIMIT;
     }
-    i64_to_i32_kernel<<<(unsigned)((nnode + 1 + 255) / 256), 256, 0, st>>>(nbrc, node_nbr_ptr, nnode + 1);
-    FL_LAUNCH_CHECK();
-    FL_HIP_CHECK(hipStreamSynchronize(st));
     *node_nnz = total;
     *max_degree = hflags[2];
     return 0;
@@ -437,18 +661,20 @@ int fl_pattern_fill(const int32_t *elements, int64_t nelem, int32_t npe, int64_t
         set_error("fl_pattern_fill: invalid argument");
         return FL_E_ARG;
     }
-    int32_t *flag = nullptr;
-    FL_HIP_CHECK(hipMallocAsync(reinterpret_cast<void **>(&flag), sizeof(int32_t), st));
-    FL_HIP_CHECK(hipMemsetAsync(flag, 0, sizeof(int32_t), st));
-    fill_neighbours_kernel<<<(unsigned)nnode, NB_T, 0, st>>>(elements, npe, node_elem_ptr, node_elem, nnode,
-                                                             node_nbr_ptr, node_nbrs, indptr, indices, flag);
+    // the last entry of indptr carries the kernels' flag to the host: FILL_BAD, or the total
+    int32_t *last = indptr + 3 * nnode;
+    FL_HIP_CHECK(hipMemsetAsync(last, 0, sizeof(int32_t), st));
+    wave_neighbours_kernel<true><<<(unsigned)((nnode + 3) / 4), 256, 0, st>>>(
+        elements, npe, node_elem_ptr, node_elem, nnode, nullptr, node_nbr_ptr, node_nbrs, indptr, indices);
+    group_neighbours_kernel<true><<<group_grid(nnode), NB_T, 0, st>>>(elements, npe, node_elem_ptr, node_elem, nnode,
+                                                                     nullptr, last, node_nbr_ptr, node_nbrs,
+                                                                     indptr, indices);
     FL_LAUNCH_CHECK();
     int32_t h = 0;
-    FL_HIP_CHECK(hipMemcpyAsync(&h, flag, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-    FL_HIP_CHECK(hipFreeAsync(flag, st));
+    FL_HIP_CHECK(hipMemcpyAsync(&h, last, sizeof(int32_t), hipMemcpyDeviceToHost, st));
     FL_HIP_CHECK(hipStreamSynchronize(st));
-    if (h) {
-        set_error("fl_pattern_fill: neighbour lists inconsistent with fl_pattern_graph (flag %d)", h);
+    if (h < 0) {
+        set_error("fl_pattern_fill: neighbour lists inconsistent with fl_pattern_graph");
         return FL_E_ARG;
     }
     return 0;
@@ -553,42 +779,31 @@ int fl_pattern_gather_plan(const int32_t *node_nbr_ptr, int64_t nnode, int32_t *
         set_error("fl_pattern_gather_plan: invalid argument");
         return FL_E_ARG;
     }
-    // class 0: the nodes of the smallest neighbour count (in meshes with element-interior
-    // nodes, exactly those: a node of two distinct elements has more neighbours than an
-    // element has nodes); classes 1.. by the limits
-    static const int32_t limits[FL_GATHER_BUCKETS] = {0, 128, 256, 512, 1024, 2048};
-    std::vector<int32_t> ptr((size_t)nnode + 1);
-    FL_HIP_CHECK(hipMemcpyAsync(ptr.data(), node_nbr_ptr, sizeof(int32_t) * (nnode + 1), hipMemcpyDeviceToHost, st));
-    FL_HIP_CHECK(hipStreamSynchronize(st));
-    int32_t dmin = INT32_MAX;
-    for (int64_t a = 0; a < nnode; ++a) dmin = std::min(dmin, ptr[a + 1] - ptr[a]);
-    std::vector<int32_t> cls((size_t)nnode);
-    int64_t count[FL_GATHER_BUCKETS] = {};
-    for (int b = 0; b < FL_GATHER_BUCKETS; ++b) bucket_degree[b] = 0;
-    for (int64_t a = 0; a < nnode; ++a) {
-        const int32_t d = ptr[a + 1] - ptr[a];
-        int b = 0;
-        if (d != dmin) {
-            b = 1;
-            while (b < FL_GATHER_BUCKETS && d > limits[b]) ++b;
-        }
-        if (b == FL_GATHER_BUCKETS) {
-            set_error("fl_pattern_gather_plan: node %lld has %d neighbours (limit %d)", (long long)a, d,
-                      limits[FL_GATHER_BUCKETS - 1]);
-            return FL_E_LIMIT;
-        }
-        cls[a] = b;
-        ++count[b];
-        if (d > bucket_degree[b]) bucket_degree[b] = d;
+    const int64_t nchunk = (nnode + PL_CHUNK - 1) / PL_CHUNK;
+    const size_t bytes = sizeof(int32_t) * (size_t)(PL_HEAD + PL_C * nchunk);
+    int32_t *w = nullptr, h[PL_HEAD];
+    FL_HIP_CHECK(hipMallocAsync(reinterpret_cast<void **>(&w), bytes, st));
+    hipError_t e = hipMemsetAsync(w, 0, bytes, st);
+    if (e == hipSuccess) {
+        plan_min_kernel<<<(unsigned)((nnode + 255) / 256), 256, 0, st>>>(node_nbr_ptr, nnode, w);
+        plan_chunk_kernel<false><<<(unsigned)nchunk, 256, 0, st>>>(node_nbr_ptr, nnode, w, nullptr);
+        plan_scan_kernel<<<1, 64 * PL_C, 0, st>>>(w, nchunk);
+        plan_chunk_kernel<true><<<(unsigned)nchunk, 256, 0, st>>>(node_nbr_ptr, nnode, w, node_order);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpyAsync(h, w, sizeof(h), hipMemcpyDeviceToHost, st);
+    (void)hipFreeAsync(w, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    FL_HIP_CHECK(e);
+    if (h[13] > 0) {
+        set_error("fl_pattern_gather_plan: a node has %d neighbours (limit %d)", h[13], 64 << (PL_C - 1));
+        return FL_E_LIMIT;
     }
     bucket_offsets[0] = 0;
-    for (int b = 0; b < FL_GATHER_BUCKETS; ++b) bucket_offsets[b + 1] = bucket_offsets[b] + (int32_t)count[b];
-    std::vector<int32_t> order((size_t)nnode);
-    int64_t cur[FL_GATHER_BUCKETS];
-    for (int b = 0; b < FL_GATHER_BUCKETS; ++b) cur[b] = bucket_offsets[b];
-    for (int64_t a = 0; a < nnode; ++a) order[cur[cls[a]]++] = (int32_t)a;
-    FL_HIP_CHECK(hipMemcpyAsync(node_order, order.data(), sizeof(int32_t) * nnode, hipMemcpyHostToDevice, st));
-    FL_HIP_CHECK(hipStreamSynchronize(st));
+    for (int b = 0; b < PL_C; ++b) {
+        bucket_offsets[b + 1] = bucket_offsets[b] + h[7 + b];
+        bucket_degree[b] = h[1 + b];
+    }
     return 0;
 }
 
