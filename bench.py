@@ -64,8 +64,8 @@ SF_KERNELS = {
        "one type per reduction)",
 }
 SF_KERNELS[2] = SF_KERNELS[4] = SF_KERNELS[0]
-DIRECT_KERNEL = ("stiffness_sf_mfma2_kernel<5,6,true> (sum-factorised: zeta on the FP64 VALU, eta and beta on "
-                 "FP64 MFMA, two types per reduction; writes the CSR itself, one launch per element colour)")
+DIRECT_KERNEL = ("stiffness_rows_kernel<5,6> (sum-factorised: zeta on the FP64 VALU, eta and beta on FP64 MFMA, "
+                 "three blocks of an element per workgroup; writes the CSR itself, one launch per element colour)")
 
 
 def direct_scatter_bytes(nelem, npe, G, nnz, table_bytes):

@@ -429,6 +429,7 @@ __global__ __launch_bounds__(256) void qp_kernel(MatParams mp0, const double *__
 #include "fl_stiffness.hpp"
 #include "fl_stiffness_bf16.hpp"
 #include "fl_stiffness_sf.hpp"
+#include "fl_stiffness_rows.hpp"
 #include "fl_mg_galerkin.hpp"
 #include "fl_mg_mf.hpp"
 namespace fl {
@@ -895,7 +896,7 @@ static int launch_galerkin_sf(int npe_c, int G, const double *qp, const int32_t 
     const dim3 grid((unsigned)groups);
 #define FL_GSF_CASE(P, QQ)                                                                                   \
     if (npe_c == P * P * P && G == QQ * QQ * QQ) {                                                         \
-        stiffness_sf_mfma2_kernel<P, QQ, false, double, double>                                            \
+        stiffness_sf_mfma2_kernel<P, QQ, double, double>                                                   \
             <<<grid, 256, 0, st>>>(qp, basis_c, nelem, Kc, nullptr, nullptr);                               \
         FL_LAUNCH_CHECK();                                                                                 \
         return 0;                                                                                          \
@@ -924,7 +925,7 @@ static int launch_stiffness_sf32(int npe, int G, const double *qp, const void *b
     const int32_t *b = static_cast<const int32_t *>(basis);
 #define FL_SF_CASE(P, QQ)                                                                                      \
     if (npe == P * P * P && G == QQ * QQ * QQ) {                                                               \
-        stiffness_sf_mfma2_kernel<P, QQ, false, float, double><<<grid, 256, 0, st>>>(qp, b, nelem, Ke, nullptr, nullptr); \
+        stiffness_sf_mfma2_kernel<P, QQ, float, double><<<grid, 256, 0, st>>>(qp, b, nelem, Ke, nullptr, nullptr); \
         FL_LAUNCH_CHECK();                                                                                     \
         return 0;                                                                                              \
     }
@@ -939,7 +940,7 @@ static int launch_stiffness_sf32(int npe, int G, const double *qp, const void *b
 }
 
 // The factorised stiffness straight into the CSR, one launch per colour in colour order
-// (stiffness_sf_mfma2_kernel's DIRECT form).  offsets (host): the colour ranges of elems.
+// (stiffness_rows_kernel).  offsets (host): the colour ranges of elems.
 // CT: the contraction type (double; float for the FP32 tangent), VT: the CSR values'
 // (double; float for FL_PREC_CSR32 with the FP32 tangent).
 template <typename CT, typename VT>
@@ -950,25 +951,38 @@ static int launch_stiffness_direct(int npe, int G, const double *qp, const void 
     for (int c = 0; c < ncolour; ++c) {
         const int64_t n = offsets[c + 1] - offsets[c];
         if (n <= 0) continue;
-        if ((n + 7) / 8 * 8 * 9 > (int64_t)INT32_MAX) {
-            set_error("too many elements of one colour for one launch");
-            return FL_E_LIMIT;
-        }
-        const dim3 grid((unsigned)((n + 7) / 8 * 8 * 9));
         const int32_t *el = elems + offsets[c];
-#define FL_SF_CASE(P, QQ)                                                                              \
-    if (npe == P * P * P && G == QQ * QQ * QQ) {                                                       \
-        stiffness_sf_mfma2_kernel<P, QQ, true, CT, VT><<<grid, 256, 0, st>>>(qp, b, n, nullptr, nullptr, V, el, \
-                                                                             elements, indptr, scat);  \
-        FL_LAUNCH_CHECK();                                                                             \
-        continue;                                                                                      \
+        // SW waves a slice, at least OCC waves a SIMD (fl_stiffness_rows.hpp).  p <= 2: a wave a
+        // slice fits (us, shared by 4 waves -> a wave each: p = 1, 20^3 172 -> 109).  p = 3: the
+        // slices' own T1 and T2 leave too few workgroups on a CU (17^3: 944 -> shared 862).
+        // p = 4: five slices do not fit in LDS; FP64 takes 4 waves (8 spill at the 128 registers
+        // that two workgroups leave each: 16^3 3840 against 2613), FP32 8 (4^3 98 against 109,
+        // 16^3 within 2 %, and 4 spill where float sums go to double values).
+        // split, a workgroup a slice: where three workgroups an element are fewer than two a CU.
+        // It repeats the loads and tables for every slice and pays where the chip is idle
+        // (together -> split: p = 4, 4^3 458 -> 148, 8^3 577 -> 467; p = 3, 10^3 216 -> 190),
+        // not where it is full (p = 4, 12^3 with 216 elements a colour 1312 -> 1355, 16^3
+        // 2613 -> 2915; p = 3, 17^3 861 -> 884)
+#define FL_ROWS_CASE(P, QQ, SW, OCC)                                                                                \
+    if (npe == P * P * P && G == QQ * QQ * QQ) {                                                                    \
+        const int split = SW > 1 && 3 * n < 2 * 256 ? 1 : 0;                                                     \
+        const int64_t groups = (n + 7) / 8 * 8 * 3 * (split ? P : 1);                                               \
+        if (groups > (int64_t)INT32_MAX) {                                                                          \
+            set_error("too many elements of one colour for one launch");                                            \
+            return FL_E_LIMIT;                                                                                      \
+        }                                                                                                           \
+        stiffness_rows_kernel<P, QQ, SW, OCC, CT, VT><<<(unsigned)groups, SW == 1 ? 64 * P : 64 * SW, 0, st>>>(     \
+            qp, b, n, V, el, elements, indptr, scat, split);                                                        \
+        FL_LAUNCH_CHECK();                                                                                          \
+        continue;                                                                                                   \
     }
-        FL_SF_CASE(2, 2)
-        FL_SF_CASE(3, 3)
-        FL_SF_CASE(4, 4)
-        FL_SF_CASE(5, 5)
-        FL_SF_CASE(5, 6)
-#undef FL_SF_CASE
+        constexpr int SW4 = sizeof(CT) == 8 ? 4 : 8, OCC4 = sizeof(CT) == 8 ? 2 : 4;
+        FL_ROWS_CASE(2, 2, 1, 4)
+        FL_ROWS_CASE(3, 3, 1, 4)
+        FL_ROWS_CASE(4, 4, 4, 3)
+        FL_ROWS_CASE(5, 5, SW4, OCC4)
+        FL_ROWS_CASE(5, 6, SW4, OCC4)
+#undef FL_ROWS_CASE
         set_error("no sum-factorised kernel for %d nodes and %d points", npe, G);
         return FL_E_ARG;
     }

@@ -353,6 +353,33 @@ def test_direct_scatter_equals_gather(cuda, p, n):
     assert np.array_equal(T, Tg)
 
 
+@pytest.mark.parametrize("p,n", [(1, 1), (2, 11), (3, 1), (3, 11), (4, 1), (4, 11)])
+def test_direct_scatter_small_and_large_colours(cuda, p, n):
+    """The direct scatter equals the gather over stored blocks where every colour is one
+    element, and where one assembly has colours on both sides of the size below which
+    a slice is a workgroup of its own (11^3 elements: parity classes of 125 to 216).  FP64
+    and FP32 blocks summed in FP64: 1e-13 (sums in another order); FP32 values: at most
+    8 roundings of a sum (8 x 2^-24)."""
+    import torch
+    from florence_amd.assembly import DeviceMeshData, assemble_device
+    m = cube_mesh("hex", p, n, jitter=0.05, seed=p)
+    fs = function_space(m, p)
+    mat = NeoHookean(3, mu=1.0, lamb=10.0)
+    x = deformed(m.points, 0.03 / n, seed=51 + p)
+    dm = DeviceMeshData(m, fs)
+    assert dm.scatter is not None
+    for kw, tol in (({}, 1e-13), ({"precision": "fp32"}, 1e-13), ({"precision": "fp32", "csr": "fp32"}, 4.8e-7)):
+        V, T, st = assemble_device(dm, mat, x, **kw)
+        V, T = V.to(torch.float64, copy=True), T.clone()
+        assert int(st[0].item()) == 0
+        kw = {k: v for k, v in kw.items() if k != "csr"}
+        Vg, Tg, _ = assemble_device(dm, mat, x, direct=False, **kw)
+        err = float((V - Vg).abs().max() / Vg.abs().max())
+        print("p={} n={} {}: |dV|/|V| = {:.2e}".format(p, n, kw, err), flush=True)
+        assert err <= tol
+        assert torch.equal(T, Tg)
+
+
 @pytest.mark.parametrize("shape", ["cube, shuffled elements", "cylinder"])
 def test_direct_scatter_irregular(cuda, shape):
     """The direct scatter on colourings that are not the 2 x 2 x 2 parity classes: a
