@@ -217,11 +217,12 @@ __global__ void transpose_jm_kernel(const double *__restrict__ Jm, int npe, int 
 // emitC: store, in place of each pair's D^{ik}, the tensor C^{ik}_{mn} = sum_{jl}
 // (dxi_m/dx_j) D^{ik}_{jl} (dxi_n/dx_l) that the sum-factorised stiffness contracts
 // (computed once per point instead of in each of the element's block workgroups).
+// fused: the caller contracts the tractions from out, and the record leaves out detJ sigma
+// and detJ.
 template <bool TANGENT, bool GEN = false>
 __device__ __forceinline__ void qp_point(const MatParams &mp, const double (&PX)[9], const double (&Px)[9], double wg,
                                          int update, bool valid, double *__restrict__ rec, int fs,
-                                         int32_t *__restrict__ status, bool emitC = false,
-                                         double *__restrict__ out = nullptr) {
+                                         int32_t *__restrict__ status, bool emitC, bool fused, double (&out)[15]) {
     double iX[9], ix[9];
     const double detX = invdet3x3(PX, iX);
     const double detx = invdet3x3(Px, ix);
@@ -283,19 +284,16 @@ __device__ __forceinline__ void qp_point(const MatParams &mp, const double (&PX)
         atomicOr(status, (m_np ? FL_S_NONPOSITIVE_J : 0) | (m_nf ? FL_S_NONFINITE : 0));
         atomicAdd(status + 1, (int)__popcll(m_np));
     }
-    if (!valid) return;
-    if (out) {
-        // dxi/dx and detJ sigma (s00 s11 s22 s01 s02 s12) for a fused traction
+    // dxi/dx and detJ sigma (s00 s11 s22 s01 s02 s12) for a fused traction
 #pragma unroll
-        for (int i = 0; i < 9; ++i) out[i] = ix[i];
-        out[9] = detJ * sig[0];
-        out[10] = detJ * sig[4];
-        out[11] = detJ * sig[8];
-        out[12] = detJ * sig[1];
-        out[13] = detJ * sig[2];
-        out[14] = detJ * sig[5];
-    }
-    if (!rec) return;
+    for (int i = 0; i < 9; ++i) out[i] = ix[i];
+    out[9] = detJ * sig[0];
+    out[10] = detJ * sig[4];
+    out[11] = detJ * sig[8];
+    out[12] = detJ * sig[1];
+    out[13] = detJ * sig[2];
+    out[14] = detJ * sig[5];
+    if (!valid || !rec) return;
     if (TANGENT) {
         // dxi/dx: read by the dense contractions (the C tensors already hold it)
         if (!emitC) {
@@ -343,7 +341,7 @@ __device__ __forceinline__ void qp_point(const MatParams &mp, const double (&PX)
                 for (int t = 0; t < 9; ++t) rec[(Q_D + 9 * p + t) * fs] = D[t];
             }
         }
-        if (!out) {
+        if (!fused) {
             // read by the traction kernels (a fused traction has them already)
             rec[(Q_S + 0) * fs] = detJ * sig[0];
             rec[(Q_S + 1) * fs] = detJ * sig[4];
@@ -419,8 +417,9 @@ __global__ __launch_bounds__(256) void qp_kernel(MatParams mp0, const double *__
         }
     }
     if (!valid) PX[0] = PX[4] = PX[8] = Px[0] = Px[4] = Px[8] = 1.0;
+    double pv[15];
     qp_point<TANGENT, GEN>(mp, PX, Px, valid ? w[g] : 1.0, update, valid,
-                           qp + e * (int64_t)G * (TANGENT ? QS : QS_RES) + g, G, status);
+                           qp + e * (int64_t)G * (TANGENT ? QS : QS_RES) + g, G, status, false, false, pv);
 }
 
 // ------------------------------------------------------------------ phase 2
@@ -999,12 +998,13 @@ static int launch_qp_sf(const MatParams &mp, const double *points, const int32_t
     const int32_t *b = static_cast<const int32_t *>(basis);
 #define FL_QSF_CASE(P, QQ)                                                                                     \
     if (npe == P * P * P && G == QQ * QQ * QQ) {                                                               \
+        const unsigned grid = (unsigned)((nelem + QpSf<P, QQ>::EPB - 1) / QpSf<P, QQ>::EPB);                   \
         if (general_law(mp.material))                                                                          \
-            qp_sf_kernel<P, QQ, TANGENT, true><<<(unsigned)nelem, 256, 0, st>>>(                               \
+            qp_sf_kernel<P, QQ, TANGENT, true><<<grid, QpSf<P, QQ>::NT, 0, st>>>(                    \
                 mp, points, elements, Eulerx, b, w, nelem, update, qp, status, elem_mat, mat_table, emitC, te,  \
                 node_elem_ptr, Tdirect);                                                                       \
         else                                                                                                   \
-            qp_sf_kernel<P, QQ, TANGENT, false><<<(unsigned)nelem, 256, 0, st>>>(                              \
+            qp_sf_kernel<P, QQ, TANGENT, false><<<grid, QpSf<P, QQ>::NT, 0, st>>>(                   \
                 mp, points, elements, Eulerx, b, w, nelem, update, qp, status, elem_mat, mat_table, emitC, te,  \
                 node_elem_ptr, Tdirect);                                                                       \
         FL_LAUNCH_CHECK();                                                                                     \

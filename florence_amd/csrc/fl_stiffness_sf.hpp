@@ -46,64 +46,6 @@ struct SfLayout {
     static constexpr int INTS = 4 + Q3 + 2 * N3 + (Q3 % 2);   // 8-byte aligned
 };
 
-// Element tractions t_(a,i) = sum_q sum_m dN_a/dxi_m (q) P[q][m][i] from the point
-// tensors P[3 m + i][t] (tensor point t) in LDS: contracted zeta, eta, beta in turn for the
-// nine (m, i), one workgroup per element.  U1 [9][P1][Q^2] and U2 [9][PP][Q] are LDS
-// work areas; U2 may share P's space (P's last reads precede the barrier before U2 is
-// written).  te in local node order; with T, a node of this element only gets its T
-// entry directly (as 0.0 + value, the accumulated form).
-template <int P1, int Q>
-__device__ __forceinline__ void traction_sf_contract(const double (&sF)[3][2][P1][Q], const double *sP,
-                                                     double *sU1, double *sU2, const int32_t *__restrict__ basis,
-                                                     int64_t e, double *__restrict__ te,
-                                                     const int32_t *__restrict__ elements,
-                                                     const int32_t *__restrict__ node_elem_ptr,
-                                                     double *__restrict__ T) {
-    typedef SfLayout<P1, Q> L;
-    constexpr int Q3 = L::Q3, N3 = L::N3, PP = L::PP;
-    constexpr int NT = 256;
-    const int tid = threadIdx.x;
-    const int32_t *loc = basis + 4 + Q3;
-    for (int t = tid; t < 9 * P1 * Q * Q; t += NT) {
-        const int mi = t / (P1 * Q * Q), r = t - mi * P1 * Q * Q;
-        const int az = r / (Q * Q), qe = (r / Q) % Q, qb = r % Q;
-        const double *f = sF[0][mi / 3 == 0][az];
-        const double *p = sP + mi * Q3 + (qb * Q + qe) * Q;
-        double s = 0.0;
-#pragma unroll
-        for (int qz = 0; qz < Q; ++qz) s += f[qz] * p[qz];
-        sU1[(mi * P1 + az) * Q * Q + qe * Q + qb] = s;
-    }
-    __syncthreads();
-    for (int t = tid; t < 9 * PP * Q; t += NT) {
-        const int mi = t / (PP * Q), r = t - mi * PP * Q;
-        const int ae = r / (P1 * Q), az = (r / Q) % P1, qb = r % Q;
-        const double *f = sF[1][mi / 3 == 1][ae];
-        double s = 0.0;
-#pragma unroll
-        for (int qe = 0; qe < Q; ++qe) s += f[qe] * sU1[(mi * P1 + az) * Q * Q + qe * Q + qb];
-        sU2[(mi * PP + ae * P1 + az) * Q + qb] = s;
-    }
-    __syncthreads();
-    for (int t = tid; t < 3 * N3; t += NT) {
-        const int tn = t / 3, i = t - 3 * tn;
-        const int ab = tn / PP, aeaz = tn - ab * PP;
-        double s = 0.0;
-#pragma unroll
-        for (int m = 0; m < 3; ++m) {
-            const double *f = sF[2][m == 2][ab];
-#pragma unroll
-            for (int qb = 0; qb < Q; ++qb) s += f[qb] * sU2[((3 * m + i) * PP + aeaz) * Q + qb];
-        }
-        const int lt = min(max(loc[tn], 0), N3 - 1);
-        te[e * 3 * N3 + 3 * lt + i] = s;
-        if (T) {
-            const int32_t a = elements[e * N3 + lt];
-            if (node_elem_ptr[a + 1] - node_elem_ptr[a] == 1) T[3 * (int64_t)a + i] = 0.0 + s;
-        }
-    }
-}
-
 // P[3 m + i] = sum_j (dxi_m/dx_j) (detJ sigma)_ij of one point from dxi/dx (9) and detJ
 // sigma (s00 s11 s22 s01 s02 s12)
 __device__ __forceinline__ void traction_point_tensor(const double *ix, const double *S, double (&P)[9]) {
@@ -114,22 +56,49 @@ __device__ __forceinline__ void traction_point_tensor(const double *ix, const do
         for (int i = 0; i < 3; ++i) P[3 * m + i] = ix[m] * Si[i][0] + ix[3 + m] * Si[i][1] + ix[6 + m] * Si[i][2];
 }
 
-// Phase 1 for tensor-product hexes: one workgroup per element.  The element's X and x
-// are staged in LDS in tensor node order and the parent Jacobians at all points,
-// dX_c/dxi_m = sum_a dN_a/dxi_m X_a,c, are contracted one direction at a time:
+// Phase 1 for tensor-product hexes: a workgroup of 128 threads (256 for 6^3 points) for the
+// EPB elements whose points fill it, a point per thread.  The elements' X and x are staged in LDS in tensor
+// node order and the parent Jacobians at all points, dX_c/dxi_m = sum_a dN_a/dxi_m X_a,c,
+// are contracted one direction at a time:
 //
 //     A[f][s0][ab,ae][qz]   = sum_az T0^{s0}[az][qz] X_f[ab,ae,az]
 //     B[f][m][ab][qe,qz]    = sum_ae T1^{[m=1]}[ae][qe] A[f][[m=0]][ab,ae][qz]
 //     P[f][m][qb,qe,qz]     = sum_ab T2^{[m=2]}[ab][qb] B[f][m][ab][qe,qz]
 //
-// (f = X_0..2, x_0..2; X then x, one pass each), then each point runs qp_point.  Same
-// records as qp_kernel, to rounding (the node sum is taken in another order).  LDS:
-// the staging shares its space with B, A with P.  With te given, the element tractions
-// follow in the same workgroup (traction_sf_contract: the point tensors in the P area,
-// the zeta results in the B area, the eta results in the P area again), and the
-// records -- if qp is given at all -- omit detJ sigma and detJ.
+// (f = X_0..2, x_0..2: A for all six, then B and P for X and for x), then each point runs
+// qp_point.  Same records as qp_kernel, to rounding (the node sum is taken in another
+// order).  With te given, the element tractions
+// t_(a,i) = sum_q sum_m dN_a/dxi_m (q) P[q][m][i] follow in the same workgroup: the point
+// tensors contracted zeta, eta, beta in turn for the nine (m, i); the records -- if qp is
+// given at all -- then omit detJ sigma and detJ.  te in local node order; with T, a node of
+// one element only gets its T entry directly (as 0.0 + value, the accumulated form).
+//
+// A task is a line: a thread reads the line's values once, forms every output of the
+// contraction with them in registers and takes the 1D basis, the same for a whole wave,
+// from scalar registers; only P's basis depends on the thread's point.  LDS strides are odd
+// where the lanes of an access step over a line.  Bound by VALU issue and LDS together
+// (p = 4, 6^3 points: 1004 VALU and 163 LDS instructions a wave, half the cycles each); a
+// task an output, which reads both factors of every product from LDS, and a workgroup an
+// element at every p were LDS-bound, and idle at small p.  Residual pass before -> now: p = 4,
+// 20^3 elements 229 -> 133 us, p = 2, 25^3 89 -> 44, p = 1, 20^3 37 -> 27; the point phase of
+// the assembly: 352 -> 284, 182 -> 67, 77 -> 26.  Two points a thread, for half of P's reads,
+// do not pay (134, and 617 for the tangent, whose registers then spill).
+typedef const double __attribute__((address_space(4))) ConstDouble;
+
+template <int P1, int Q>
+struct QpSf {
+    typedef SfLayout<P1, Q> L;
+    static constexpr int NT = L::Q3 <= 128 ? 128 : 256, QQ = Q * Q, EPB = NT / L::Q3;
+    static constexpr int XS = P1 | 1, AS = Q | 1, PS = QQ | 1;   // line strides in LDS
+    static constexpr int SZ_X = 6 * L::PP * XS, SZ_B = 9 * P1 * QQ;          // U1 [9][P1][QQ] in B's space
+    static constexpr int SZ_A = 12 * L::PP * AS, SZ_P = 9 * Q * PS;          // U2 [9][PP][AS] in A's space
+    static constexpr int SZ_XB = SZ_X > SZ_B ? SZ_X : SZ_B, SZ_AP = SZ_A > SZ_P ? SZ_A : SZ_P;
+    static_assert(EPB >= 1, "one point per thread");
+    static_assert(9 * L::PP * AS <= SZ_AP, "U2 in A's space");
+};
+
 template <int P1, int Q, bool TANGENT, bool GEN>
-__global__ __launch_bounds__(256) void qp_sf_kernel(MatParams mp0, const double *__restrict__ points,
+__global__ __launch_bounds__((QpSf<P1, Q>::NT), TANGENT ? (GEN ? 2 : 3) : 4) void qp_sf_kernel(MatParams mp0, const double *__restrict__ points,
                                                     const int32_t *__restrict__ elements,
                                                     const double *__restrict__ Eulerx,
                                                     const int32_t *__restrict__ basis, const double *__restrict__ w,
@@ -140,99 +109,210 @@ __global__ __launch_bounds__(256) void qp_sf_kernel(MatParams mp0, const double 
                                                     const int32_t *__restrict__ node_elem_ptr = nullptr,
                                                     double *__restrict__ T = nullptr) {
     typedef SfLayout<P1, Q> L;
-    constexpr int Q3 = L::Q3, N3 = L::N3, PP = L::PP;
-    constexpr int NT = 256;
-    static_assert(Q3 <= NT, "one point per thread");
-    // two passes (X, then x) of three fields each keep the LDS small (~30 KB at p = 4)
-    constexpr int NF = 3;
-    constexpr int SZ_X = NF * N3, SZ_B = NF * 3 * P1 * Q * Q, SZ_A = NF * 2 * PP * Q, SZ_P = NF * 3 * Q3;
-    __shared__ double sF[3][2][P1][Q];
-    __shared__ double sXB[SZ_X > SZ_B ? SZ_X : SZ_B];
-    __shared__ double sAP[SZ_A > SZ_P ? SZ_A : SZ_P];
-    const int64_t e = blockIdx.x;
-    if (e >= nelem) return;
+    typedef QpSf<P1, Q> C;
+    constexpr int Q3 = L::Q3, N3 = L::N3, PP = L::PP, QQ = C::QQ, EPB = C::EPB, NT = C::NT;
+    constexpr int XS = C::XS, AS = C::AS, PS = C::PS, SZ_XB = C::SZ_XB, SZ_AP = C::SZ_AP;
+    __shared__ double sFb[2][P1][Q];
+    __shared__ double sXB[EPB * SZ_XB];
+    __shared__ double sAP[EPB * SZ_AP];
+    const int64_t e0 = (int64_t)blockIdx.x * EPB;
+    const int ne = (int)min((int64_t)EPB, nelem - e0);
+    if (ne <= 0) return;
     const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int32_t *g_of_t = basis + 4;
     const int32_t *loc = basis + 4 + Q3;
     const double *f1d = reinterpret_cast<const double *>(basis + L::INTS);
-    const MatParams mp = element_material(mp0, e, elem_mat, mat_table);
-    for (int t = tid; t < 3 * 2 * P1 * Q; t += NT) (&sF[0][0][0][0])[t] = f1d[t];
-    const int32_t *conn = elements + e * (int64_t)N3;
-    const bool valid = tid < Q3;
-    const int tq = valid ? tid : 0;
+    // 1D basis s (0 values, 1 derivatives) of direction d, read through scalar loads where it
+    // is used: an address the compiler cannot trace keeps it from holding all of them in
+    // registers over the whole kernel
+    const auto f = [&](int d, int s) {
+        uint64_t a = reinterpret_cast<uint64_t>(f1d + (d * 2 + s) * P1 * Q);
+        asm volatile("" : "+s"(a));
+        return reinterpret_cast<const ConstDouble *>(a);
+    };
+    for (int t = tid; t < 2 * P1 * Q; t += NT) (&sFb[0][0][0])[t] = f1d[4 * P1 * Q + t];
+    // table entries are clamped into range
+    for (int t = tid; t < ne * N3; t += NT) {
+        const int el = t / N3, tn = t - el * N3;
+        const int64_t nd = elements[(e0 + el) * N3 + min(max(loc[tn], 0), N3 - 1)];
+        double *x = sXB + el * SZ_XB + (tn / P1) * XS + tn % P1;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            x[c * PP * XS] = points[3 * nd + c];
+            x[(3 + c) * PP * XS] = Eulerx[3 * nd + c];
+        }
+    }
+    __syncthreads();
+    // A: line (element, f, ab, ae)
+    for (int t = tid; t < ne * 6 * PP; t += NT) {
+        const int el = t / (6 * PP), r = t - el * 6 * PP, fi = r / PP, abe = r - fi * PP;
+        const double *x = sXB + el * SZ_XB + r * XS;
+        double v[P1];
+#pragma unroll
+        for (int az = 0; az < P1; ++az) v[az] = x[az];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            double *a = sAP + el * SZ_AP + ((fi * 2 + s) * PP + abe) * AS;
+            const ConstDouble *l = f(0, s);
+#pragma unroll
+            for (int qz = 0; qz < Q; ++qz) {
+                double acc = 0.0;
+#pragma unroll
+                for (int az = 0; az < P1; ++az) acc += l[az * Q + qz] * v[az];
+                a[qz] = acc;
+            }
+        }
+    }
+    // this thread's point
+    const int pel = tid / Q3, tq = tid - pel * Q3;
+    const bool valid = pel < ne;
+    const int cel = valid ? pel : 0;
+    const int qb = tq / QQ, qez = tq - qb * QQ;
     double PJ[2][9];
 #pragma unroll
     for (int pass = 0; pass < 2; ++pass) {
-        // the previous pass's last reads of sXB and sAP precede the barriers below
-        const double *src = pass ? Eulerx : points;
-        for (int t = tid; t < N3; t += NT) {
-            const int64_t nd = conn[min(max(loc[t], 0), N3 - 1)];
+        __syncthreads();   // A written; the previous pass's reads of B done
+        // B: lines (element, f, ab, qz), those of A's s0 = 0 giving m = 1 and 2, those of
+        // s0 = 1 giving m = 0; a wave's lines are of one kind
+        constexpr int NW = (EPB * 3 * P1 * Q + 63) / 64;
+        for (int wt = wave; wt < 2 * NW; wt += NT / 64) {
+            const int s0 = wt >= NW;
+            const int t = (wt - s0 * NW) * 64 + lane;
+            if (t < ne * 3 * P1 * Q) {
+                const int el = t / (3 * P1 * Q), r = t - el * 3 * P1 * Q;
+                const int fi = r / (P1 * Q), ab = (r / Q) % P1, qz = r % Q;
+                const double *a = sAP + el * SZ_AP + (((3 * pass + fi) * 2 + s0) * PP + ab * P1) * AS + qz;
+                double *bo = sXB + el * SZ_XB + (fi * 3 * P1 + ab) * QQ + qz;
+                double v[P1];
 #pragma unroll
-            for (int c = 0; c < 3; ++c) sXB[c * N3 + t] = src[3 * nd + c];
+                for (int ae = 0; ae < P1; ++ae) v[ae] = a[ae * AS];
+                const auto contract = [&](int m) {
+                    const ConstDouble *l = f(1, m == 1);
+#pragma unroll
+                    for (int qe = 0; qe < Q; ++qe) {
+                        double acc = 0.0;
+#pragma unroll
+                        for (int ae = 0; ae < P1; ++ae) acc += l[ae * Q + qe] * v[ae];
+                        bo[m * P1 * QQ + qe * Q] = acc;
+                    }
+                };
+                if (s0) {
+                    contract(0);
+                } else {
+                    contract(1);
+                    contract(2);
+                }
+            }
         }
         __syncthreads();
-        // A[f][s0][(ab,ae)][qz]
-        for (int t = tid; t < SZ_A; t += NT) {
-            const int qz = t % Q, r = t / Q;
-            const int abe = r % PP, r2 = r / PP;
-            const int s0 = r2 % 2, f = r2 / 2;
-            const double *xf = sXB + f * N3 + abe * P1;
-            double acc = 0.0;
-#pragma unroll
-            for (int az = 0; az < P1; ++az) acc += sF[0][s0][az][qz] * xf[az];
-            sAP[t] = acc;
-        }
-        __syncthreads();
-        // B[f][m][ab][(qe,qz)]
-        for (int t = tid; t < SZ_B; t += NT) {
-            const int qez = t % (Q * Q), r = t / (Q * Q);
-            const int ab = r % P1, r2 = r / P1;
-            const int m = r2 % 3, f = r2 / 3;
-            const int qe = qez / Q, qz = qez % Q;
-            const double *a = sAP + ((f * 2 + (m == 0)) * PP + ab * P1) * Q + qz;
-            double acc = 0.0;
-#pragma unroll
-            for (int ae = 0; ae < P1; ++ae) acc += sF[1][m == 1][ae][qe] * a[ae * Q];
-            sXB[t] = acc;
-        }
-        __syncthreads();
-        // P[f][m][(qb,qe,qz)]
-        for (int t = tid; t < SZ_P; t += NT) {
-            const int tqq = t % Q3, r = t / Q3;
-            const int m = r % 3, f = r / 3;
-            const int qb = tqq / (Q * Q), qez = tqq % (Q * Q);
-            const double *bb = sXB + (f * 3 + m) * P1 * Q * Q + qez;
-            double acc = 0.0;
-#pragma unroll
-            for (int ab = 0; ab < P1; ++ab) acc += sF[2][m == 2][ab][qb] * bb[ab * Q * Q];
-            sAP[t] = acc;
-        }
-        __syncthreads();
+        // P at this thread's point
+        const double *bb = sXB + cel * SZ_XB + qez;
 #pragma unroll
         for (int m = 0; m < 3; ++m)
 #pragma unroll
-            for (int c = 0; c < 3; ++c) PJ[pass][3 * m + c] = sAP[(c * 3 + m) * Q3 + tq];
+            for (int c = 0; c < 3; ++c) {
+                double acc = 0.0;
+#pragma unroll
+                for (int ab = 0; ab < P1; ++ab) acc += sFb[m == 2][ab][qb] * bb[((c * 3 + m) * P1 + ab) * QQ];
+                asm volatile("" : "+v"(acc));   // summed here: its operands are not kept for later
+                PJ[pass][3 * m + c] = acc;
+            }
     }
+    const int64_t e = e0 + cel;
+    const MatParams mp = element_material(mp0, e, elem_mat, mat_table);
     const int g = min(max(g_of_t[tq], 0), Q3 - 1);
     // te given: the element tractions are contracted here from the point values, and
     // the records (qp, when given) are only what the stiffness kernels read
     double pv[15];
     qp_point<TANGENT, GEN>(mp, PJ[0], PJ[1], w[g], update, valid,
                       qp ? qp + e * (int64_t)Q3 * (TANGENT ? QS : QS_RES) + g : nullptr, Q3, status, emitC != 0,
-                      te ? pv : nullptr);
-    if (te) {
-        static_assert(9 * P1 * Q * Q <= (SZ_X > SZ_B ? SZ_X : SZ_B), "U1 in the B area");
-        static_assert(9 * PP * Q <= (SZ_A > SZ_P ? SZ_A : SZ_P) && 9 * Q3 <= (SZ_A > SZ_P ? SZ_A : SZ_P),
-                      "P and U2 in the P area");
-        __syncthreads();   // the last reads of sAP (PJ) precede
-        if (valid) {
-            double P[9];
-            traction_point_tensor(pv, pv + 9, P);
+                      te != nullptr, pv);
+    if (!te) return;
+    // A's last reads precede the barrier before the second P
+    if (valid) {
+        double P[9];
+        traction_point_tensor(pv, pv + 9, P);
+        double *po = sAP + pel * SZ_AP + (tq % Q) * PS + (tq / Q) % Q * Q + qb;
 #pragma unroll
-            for (int mi = 0; mi < 9; ++mi) sAP[mi * Q3 + tq] = P[mi];
+        for (int mi = 0; mi < 9; ++mi) po[mi * Q * PS] = P[mi];
+    }
+    __syncthreads();
+    // lines of the nine (m, i), those whose m takes the derivatives of direction D (m == D)
+    // first; a wave's lines are of one kind: task(el, mi, r, basis) of r in [0, R)
+    const auto lines = [&](int D, int R, const auto &task) {
+        const int n1 = (EPB * 3 * R + 63) / 64, n2 = (EPB * 6 * R + 63) / 64;
+        for (int wt = wave; wt < n1 + n2; wt += NT / 64) {
+            const int s = wt < n1, k = s ? 3 : 6;
+            const int t = (s ? wt : wt - n1) * 64 + lane;
+            if (t < ne * k * R) {
+                const int el = t / (k * R), r2 = t - el * k * R, j = r2 / R;
+                // m of the others: 1, 2 (D = 0) or 0, 2 (D = 1)
+                const int m = s ? D : (j < 3 ? 1 - D : 2);
+                task(el, 3 * m + j % 3, r2 - j * R, f(D, s));
+            }
         }
-        __syncthreads();
-        traction_sf_contract<P1, Q>(sF, sAP, sXB, sAP, basis, e, te, elements, node_elem_ptr, T);
+    };
+    // U1 [mi][az][qe, qb]
+    lines(0, QQ, [&](int el, int mi, int r, const ConstDouble *l) {
+        const double *p = sAP + el * SZ_AP + mi * Q * PS + r;
+        double *u = sXB + el * SZ_XB + mi * P1 * QQ + r;
+        double v[Q];
+#pragma unroll
+        for (int qz = 0; qz < Q; ++qz) v[qz] = p[qz * PS];
+#pragma unroll
+        for (int az = 0; az < P1; ++az) {
+            double acc = 0.0;
+#pragma unroll
+            for (int qz = 0; qz < Q; ++qz) acc += l[az * Q + qz] * v[qz];
+            u[az * QQ] = acc;
+        }
+    });
+    __syncthreads();
+    // U2 [mi][ae, az][qb]
+    lines(1, P1 * Q, [&](int el, int mi, int r, const ConstDouble *l) {
+        const int az = r / Q, q = r - az * Q;
+        const double *p = sXB + el * SZ_XB + (mi * P1 + az) * QQ + q;
+        double *u = sAP + el * SZ_AP + (mi * PP + az) * AS + q;
+        double v[Q];
+#pragma unroll
+        for (int qe = 0; qe < Q; ++qe) v[qe] = p[qe * Q];
+#pragma unroll
+        for (int ae = 0; ae < P1; ++ae) {
+            double acc = 0.0;
+#pragma unroll
+            for (int qe = 0; qe < Q; ++qe) acc += l[ae * Q + qe] * v[qe];
+            u[ae * P1 * AS] = acc;
+        }
+    });
+    __syncthreads();
+    for (int t = tid; t < ne * 3 * PP; t += NT) {
+        const int el = t / (3 * PP), r = t - el * 3 * PP, aeaz = r / 3, i = r - 3 * aeaz;
+        double s[P1];
+#pragma unroll
+        for (int ab = 0; ab < P1; ++ab) s[ab] = 0.0;
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+            const double *u = sAP + el * SZ_AP + ((3 * m + i) * PP + aeaz) * AS;
+            const ConstDouble *l = f(2, m == 2);
+            double v[Q];
+#pragma unroll
+            for (int q = 0; q < Q; ++q) v[q] = u[q];
+#pragma unroll
+            for (int ab = 0; ab < P1; ++ab)
+#pragma unroll
+                for (int q = 0; q < Q; ++q) s[ab] += l[ab * Q + q] * v[q];
+        }
+        const int64_t ee = e0 + el;
+#pragma unroll
+        for (int ab = 0; ab < P1; ++ab) {
+            const int lt = min(max(loc[ab * PP + aeaz], 0), N3 - 1);
+            te[ee * 3 * N3 + 3 * lt + i] = s[ab];
+            if (T) {
+                const int32_t a = elements[ee * N3 + lt];
+                if (node_elem_ptr[a + 1] - node_elem_ptr[a] == 1) T[3 * (int64_t)a + i] = 0.0 + s[ab];
+            }
+        }
     }
 }
 

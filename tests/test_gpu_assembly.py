@@ -380,6 +380,24 @@ def test_direct_scatter_small_and_large_colours(cuda, p, n):
         assert torch.equal(T, Tg)
 
 
+@pytest.mark.parametrize("p,n", [(1, 1), (1, 3), (2, 1), (2, 3), (3, 1), (3, 3), (4, 1)])
+def test_point_kernel_element_groups(cuda, p, n):
+    """The factorised point kernel takes 16, 4, 2 or 1 elements (p = 1..4) a workgroup: one
+    element, and 27, which leaves a part of the last workgroup empty.  K and T against
+    the oracle; the residual-only pass gives the same T."""
+    import torch
+    from florence_amd.assembly import residual_device
+    m = cube_mesh("hex", p, n, jitter=0.05, seed=60 + p)
+    fs = function_space(m, p)
+    mat = MooneyRivlin(3, mu1=1.0, mu2=0.7, lamb=10.0)
+    x = deformed(m.points, 0.04, seed=61 + p)
+    dm, V, T = _check(m, fs, mat, x, "element groups hex p{} n={}".format(p, n))
+    R, st = residual_device(dm, mat, x)
+    torch.cuda.synchronize()
+    assert int(st[0].item()) == 0
+    assert np.abs(R.cpu().numpy() - T).max() <= 1e-13 * np.abs(T).max()
+
+
 @pytest.mark.parametrize("shape", ["cube, shuffled elements", "cylinder"])
 def test_direct_scatter_irregular(cuda, shape):
     """The direct scatter on colourings that are not the 2 x 2 x 2 parity classes: a
