@@ -80,8 +80,9 @@ __device__ __forceinline__ void traction_point_tensor(const double *ix, const do
 // (p = 4, 6^3 points: 1004 VALU and 163 LDS instructions a wave, half the cycles each); a
 // task an output, which reads both factors of every product from LDS, and a workgroup an
 // element at every p were LDS-bound, and idle at small p.  Residual pass before -> now: p = 4,
-// 20^3 elements 229 -> 133 us, p = 2, 25^3 89 -> 44, p = 1, 20^3 37 -> 27; the point phase of
-// the assembly: 352 -> 284, 182 -> 67, 77 -> 26.  Two points a thread, for half of P's reads,
+// 20^3 elements 229 -> 125 us, p = 2, 25^3 89 -> 44, p = 1, 20^3 37 -> 29; the point phase of
+// the assembly: 352 -> 230, 182 -> 68, 77 -> 26.  A thread takes record point g, not tensor
+// point g: its wave's 54 record stores are then contiguous (p = 4, 20^3 284 -> 230).  Two points a thread, for half of P's reads,
 // do not pay (134, and 617 for the tangent, whose registers then spill).
 typedef const double __attribute__((address_space(4))) ConstDouble;
 
@@ -115,6 +116,7 @@ __global__ __launch_bounds__((QpSf<P1, Q>::NT), TANGENT ? (GEN ? 2 : 3) : 4) voi
     __shared__ double sFb[2][P1][Q];
     __shared__ double sXB[EPB * SZ_XB];
     __shared__ double sAP[EPB * SZ_AP];
+    __shared__ int16_t sTg[Q3];   // tensor point of record point g
     const int64_t e0 = (int64_t)blockIdx.x * EPB;
     const int ne = (int)min((int64_t)EPB, nelem - e0);
     if (ne <= 0) return;
@@ -133,6 +135,7 @@ __global__ __launch_bounds__((QpSf<P1, Q>::NT), TANGENT ? (GEN ? 2 : 3) : 4) voi
     };
     for (int t = tid; t < 2 * P1 * Q; t += NT) (&sFb[0][0][0])[t] = f1d[4 * P1 * Q + t];
     // table entries are clamped into range
+    for (int t = tid; t < Q3; t += NT) sTg[min(max(g_of_t[t], 0), Q3 - 1)] = (int16_t)t;
     for (int t = tid; t < ne * N3; t += NT) {
         const int el = t / N3, tn = t - el * N3;
         const int64_t nd = elements[(e0 + el) * N3 + min(max(loc[tn], 0), N3 - 1)];
@@ -164,10 +167,11 @@ __global__ __launch_bounds__((QpSf<P1, Q>::NT), TANGENT ? (GEN ? 2 : 3) : 4) voi
             }
         }
     }
-    // this thread's point
-    const int pel = tid / Q3, tq = tid - pel * Q3;
+    // this thread's point: record point g, so that a wave's record stores are contiguous
+    const int pel = tid / Q3, g = tid - pel * Q3;
     const bool valid = pel < ne;
     const int cel = valid ? pel : 0;
+    const int tq = min(max((int)sTg[g], 0), Q3 - 1);
     const int qb = tq / QQ, qez = tq - qb * QQ;
     double PJ[2][9];
 #pragma unroll
@@ -221,7 +225,6 @@ __global__ __launch_bounds__((QpSf<P1, Q>::NT), TANGENT ? (GEN ? 2 : 3) : 4) voi
     }
     const int64_t e = e0 + cel;
     const MatParams mp = element_material(mp0, e, elem_mat, mat_table);
-    const int g = min(max(g_of_t[tq], 0), Q3 - 1);
     // te given: the element tractions are contracted here from the point values, and
     // the records (qp, when given) are only what the stiffness kernels read
     double pv[15];
