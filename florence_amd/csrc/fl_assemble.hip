@@ -998,13 +998,13 @@ static int launch_qp_sf(const MatParams &mp, const double *points, const int32_t
     const int32_t *b = static_cast<const int32_t *>(basis);
 #define FL_QSF_CASE(P, QQ)                                                                                     \
     if (npe == P * P * P && G == QQ * QQ * QQ) {                                                               \
-        const unsigned grid = (unsigned)((nelem + QpSf<P, QQ>::EPB - 1) / QpSf<P, QQ>::EPB);                   \
+        const unsigned grid = (unsigned)((nelem + SfLines<P, QQ, 6>::EPB - 1) / SfLines<P, QQ, 6>::EPB);                   \
         if (general_law(mp.material))                                                                          \
-            qp_sf_kernel<P, QQ, TANGENT, true><<<grid, QpSf<P, QQ>::NT, 0, st>>>(                    \
+            qp_sf_kernel<P, QQ, TANGENT, true><<<grid, SfLines<P, QQ, 6>::NT, 0, st>>>(                    \
                 mp, points, elements, Eulerx, b, w, nelem, update, qp, status, elem_mat, mat_table, emitC, te,  \
                 node_elem_ptr, Tdirect);                                                                       \
         else                                                                                                   \
-            qp_sf_kernel<P, QQ, TANGENT, false><<<grid, QpSf<P, QQ>::NT, 0, st>>>(                   \
+            qp_sf_kernel<P, QQ, TANGENT, false><<<grid, SfLines<P, QQ, 6>::NT, 0, st>>>(                   \
                 mp, points, elements, Eulerx, b, w, nelem, update, qp, status, elem_mat, mat_table, emitC, te,  \
                 node_elem_ptr, Tdirect);                                                                       \
         FL_LAUNCH_CHECK();                                                                                     \
@@ -1283,19 +1283,19 @@ int mf_round_records(const MfOp &op, float *c32, hipStream_t st) {
 }
 
 int mf_element_apply(const MfOp &op, const uint8_t *free_mask, const double *x, hipStream_t st) {
-    const int64_t chunk = (op.nelem + 7) / 8;
-    const unsigned grid = (unsigned)(8 * chunk);
 #define FL_MF_LAUNCH(P, QQ)                                                                                        \
     do {                                                                                                           \
+        constexpr int EPB = SfLines<P, QQ, 3>::EPB, NT = SfLines<P, QQ, 3>::NT;                                    \
+        const unsigned grid = (unsigned)(8 * (((op.nelem + EPB - 1) / EPB + 7) / 8));                              \
         if (op.c16)                                                                                                \
-            mf_element_kernel<P, QQ, 2><<<grid, 256, 0, st>>>(op.qp, op.c32, op.c16, op.basis, op.elements,         \
-                                                              op.nelem, free_mask, x, op.ye);                      \
+            mf_element_kernel<P, QQ, 2><<<grid, NT, 0, st>>>(op.qp, op.c32, op.c16, op.basis, op.elements,         \
+                                                             op.nelem, free_mask, x, op.ye);                       \
         else if (op.c32)                                                                                           \
-            mf_element_kernel<P, QQ, 1><<<grid, 256, 0, st>>>(op.qp, op.c32, op.c16, op.basis, op.elements,         \
-                                                              op.nelem, free_mask, x, op.ye);                      \
+            mf_element_kernel<P, QQ, 1><<<grid, NT, 0, st>>>(op.qp, op.c32, op.c16, op.basis, op.elements,         \
+                                                             op.nelem, free_mask, x, op.ye);                       \
         else                                                                                                       \
-            mf_element_kernel<P, QQ, 0><<<grid, 256, 0, st>>>(op.qp, op.c32, op.c16, op.basis, op.elements,         \
-                                                              op.nelem, free_mask, x, op.ye);                      \
+            mf_element_kernel<P, QQ, 0><<<grid, NT, 0, st>>>(op.qp, op.c32, op.c16, op.basis, op.elements,         \
+                                                             op.nelem, free_mask, x, op.ye);                       \
     } while (0)
     if (op.p1 == 2 && op.q == 2)
         FL_MF_LAUNCH(2, 2);

@@ -6,260 +6,103 @@
 // the point weight included),
 //     y_{a,i} = sum_q sum_m dN_a/dxi_m(q) S_{im}(q),
 //     S_{im}  = sum_{k,n} C^{ik}_{mn}(q) G_{kn}(q),   G_{kn} = sum_b dN_b/dxi_n(q) x_{b,k},
-// with dN_b/dxi_n = prod_d T_d^{[d == n]}[b_d][q_d] (T^0 = l, T^1 = l'; d = zeta, eta,
-// beta; tensor node (ab P1 + ae) P1 + az, tensor point (qb Q + qe) Q + qz).  The gradients
-// are three one-direction contractions,
-//   U1[k][sb][qb][ae,az]  = sum_ab T_b^sb[ab][qb] x_k[ab,ae,az]                    sb = 0, 1
-//   U2[k][n][qb][qe][az]  = sum_ae T_e^se[ae][qe] U1[k][sb][qb][ae,az]   n: (sb, se) = (0,0) (0,1) (1,0)
-//   G[k][n][qb,qe,qz]     = sum_az T_z^{[n = 0]}[az][qz] U2[k][n][qb][qe][az]
-// and the transposed sum runs them backwards:
-//   W[i][m][qb][qe][az]   = sum_qz T_z^{[m = 0]}[az][qz] S[i][m][qb,qe,qz]
-//   Z[i][sb][qb][ae,az]   = sum_qe (sb = 0: T_e^0 W[i][0] + T_e^1 W[i][1]; sb = 1: T_e^0 W[i][2])
-//   y[i][ab,ae,az]        = sum_qb T_b^0[ab][qb] Z[i][0] + T_b^1[ab][qb] Z[i][1]
+// contracted one direction at a time with SfLines (gradients of x's three components at the
+// points, and back to the nodes).
 // About 124 kflop per p = 4 element, and the 54 C values per point read once (K_e itself
-// is 140,625 doubles).  One workgroup per element, each XCD taking a contiguous range of
-// elements (its L2 then holds the x of neighbouring elements); two LDS buffers alternate
-// between the stages (the per-point stage works in place: each thread reads its point's
-// nine gradients before it writes the nine S values over them), and each stage reads an
-// operand from LDS once per pencil, not once per multiply-add.
+// is 140,625 doubles).  Each XCD takes a contiguous range of elements (its L2 then holds the x
+// of neighbouring elements).
 #pragma once
 
 namespace fl {
 
-template <int P1, int Q>
-struct MfLayout {
-    static constexpr int N3 = P1 * P1 * P1, Q3 = Q * Q * Q, PP = P1 * P1, QQ = Q * Q;
-    static constexpr int mx(int a, int b) { return a > b ? a : b; }
-    // buffer A: x (3 N3), U2 (9 QQ P1), W (9 QQ P1); buffer B: U1 (6 Q PP), G then S (9 Q3), Z (6 Q PP)
-    static constexpr int BUFA = mx(3 * N3, 9 * QQ * P1);
-    static constexpr int BUFB = mx(6 * Q * PP, 9 * Q3);
-};
-
-// C32: the C tensors rounded to FP32 (c32 [e][54][Q3]) instead of the records; each
-// thread's 54 values are loaded into registers when the workgroup starts, so their latency
-// overlaps the gradient stages.  The BF16 form fits five workgroups per CU (LDS and
-// registers); the others four.
+// CK: 0 the FP64 records, 1 their FP32 copy, 2 their BF16 copy (c32 [e][54][Q3], c16
+// [e][27][Q3], two values a word).  The copy's values are loaded after B: loaded when the
+// workgroup starts they delay x (18.7 -> 21.1 us).  Bound by the latency of its eight stages: 1,728
+// elements of 125 nodes and 6^3 points, BF16, are 6.75 elements a CU, five at a time, each
+// about 10 us; the bytes (40 MB of C, 12 of vectors) take 10 us.  Before SfLines, with the 1D
+// basis and both buffers in LDS, 25.0 us; now 18.7.  Two points a thread and twice the
+// elements in flight: 21.2.
 template <int P1, int Q, int CK>
-__global__ __launch_bounds__(256, CK == 2 ? 5 : 4) void mf_element_kernel(const double *__restrict__ qp,
-                                                         const float *__restrict__ c32,
-                                                         const uint32_t *__restrict__ c16,
-                                                         const int32_t *__restrict__ basis,
-                                                         const int32_t *__restrict__ elements, int64_t nelem,
-                                                         const uint8_t *__restrict__ free_mask,
-                                                         const double *__restrict__ x, double *__restrict__ ye) {
-    typedef SfLayout<P1, Q> L;
-    typedef MfLayout<P1, Q> M;
-    constexpr int N3 = M::N3, Q3 = M::Q3, PP = M::PP, QQ = M::QQ, NT = 256;
-    // CK: 0 the FP64 records, 1 their FP32 copy, 2 their BF16 copy
-    constexpr bool C32 = CK != 0;
-    static_assert(!C32 || Q3 <= NT, "one point per thread");
-    __shared__ double sF[3][2][P1][Q];
-    __shared__ double sA[M::BUFA];
-    __shared__ double sB[M::BUFB];
-    __shared__ int32_t sLoc[N3];   // local node of tensor node t
-    __shared__ int16_t sT[Q3];     // tensor point of record point g
+__global__ __launch_bounds__((SfLines<P1, Q, 3>::NT), CK == 1 ? 4 : 5) void mf_element_kernel(
+    const double *__restrict__ qp, const float *__restrict__ c32, const uint32_t *__restrict__ c16,
+    const int32_t *__restrict__ basis, const int32_t *__restrict__ elements, int64_t nelem,
+    const uint8_t *__restrict__ free_mask, const double *__restrict__ x, double *__restrict__ ye) {
+    typedef SfLines<P1, Q, 3> C;
+    constexpr int Q3 = C::Q3, N3 = C::N3, EPB = C::EPB, NT = C::NT;
+    __shared__ double sFb[2][P1][Q];
+    __shared__ double sAP[C::LDS];
 
-    const int64_t chunk = (nelem + 7) / 8;
+    const int64_t chunk = ((nelem + EPB - 1) / EPB + 7) / 8;
     const int64_t k8 = blockIdx.x >> 3;
-    const int64_t e = (int64_t)(blockIdx.x & 7) * chunk + k8;
-    if (k8 >= chunk || e >= nelem) return;
+    const int64_t e0 = ((int64_t)(blockIdx.x & 7) * chunk + k8) * EPB;
+    const int ne = (int)min((int64_t)EPB, nelem - e0);
+    if (k8 >= chunk || ne <= 0) return;
     const int tid = threadIdx.x;
     const int32_t *g_of_t = basis + 4;
     const int32_t *loc = basis + 4 + Q3;
-    const double *f1d = reinterpret_cast<const double *>(basis + L::INTS);
-    const int32_t *conn = elements + e * N3;
-    float cr[C32 ? 54 : 1];
+    const double *f1d = reinterpret_cast<const double *>(basis + SfLayout<P1, Q>::INTS);
+    const C c = {f1d, loc, ne, tid, __builtin_amdgcn_readfirstlane(tid >> 6), tid & 63, sAP, sAP};
+    // this thread's point: table entries are clamped into range
+    const int pel = tid / Q3, u = tid - pel * Q3;
+    const bool valid = pel < ne;
+    const int cel = valid ? pel : 0;
+    const int64_t e = e0 + cel;
+    const int g = min(max(g_of_t[C::point(u)], 0), Q3 - 1);
+    for (int t = tid; t < 2 * P1 * Q; t += NT) (&sFb[0][0][0])[t] = f1d[4 * P1 * Q + t];
+    for (int t = tid; t < ne * N3; t += NT) {
+        const int el = EPB == 1 ? 0 : t / N3, tn = t - el * N3;
+        const int64_t a = elements[(e0 + el) * N3 + min(max(loc[tn], 0), N3 - 1)];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const double xv = x[3 * a + k];   // read either way: one latency, not two
+            *c.x(el, k, tn) = free_mask[3 * a + k] ? xv : 0.0;
+        }
+    }
+    __syncthreads();
+    c.form_A();
+    __syncthreads();
+    c.form_B(0);
+    // the point's values of a rounded copy, in flight over the gradient
+    float cr[CK == 1 ? 54 : 1];
+    uint32_t cw[CK == 2 ? 27 : 1];
     if constexpr (CK == 1) {
-        const float *r32 = c32 + e * (int64_t)54 * Q3 + min(tid, Q3 - 1);
 #pragma unroll
-        for (int f = 0; f < 54; ++f) cr[f] = r32[f * Q3];
+        for (int f = 0; f < 54; ++f) cr[f] = c32[(e * 54 + f) * Q3 + g];
     } else if constexpr (CK == 2) {
-        const uint32_t *r16 = c16 + e * (int64_t)27 * Q3 + min(tid, Q3 - 1);
-        uint32_t w[27];
 #pragma unroll
-        for (int j = 0; j < 27; ++j) w[j] = r16[j * Q3];
-#pragma unroll
-        for (int j = 0; j < 27; ++j) {
-            cr[2 * j] = __uint_as_float(w[j] << 16);
-            cr[2 * j + 1] = __uint_as_float(w[j] & 0xFFFF0000u);
-        }
-    }
-    for (int t = tid; t < 6 * P1 * Q; t += NT) (&sF[0][0][0][0])[t] = f1d[t];
-    for (int t = tid; t < Q3; t += NT) sT[min(max(g_of_t[t], 0), Q3 - 1)] = (int16_t)t;
-    for (int t = tid; t < N3; t += NT) {
-        const int l = min(max(loc[t], 0), N3 - 1);
-        sLoc[t] = l;
-        const int64_t a = conn[l];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) sA[k * N3 + t] = free_mask[3 * a + k] ? x[3 * a + k] : 0.0;
+        for (int f = 0; f < 27; ++f) cw[f] = c16[(e * 27 + f) * Q3 + g];
     }
     __syncthreads();
-    // Each stage runs over "pencils": a thread loads the P1 (or Q) values along the
-    // contracted direction into registers once and writes every output of its pencil.
-    // beta: U1 -> B, pencils (k, sb, ae az)
-    for (int t = tid; t < 6 * PP; t += NT) {
-        const int r = t % PP, kb = t / PP;
-        const int k = kb >> 1, sb = kb & 1;
-        double xv[P1];
+    double G[9], S[9];   // G[3 n + k], S[3 m + i]
+    c.gradient(sFb, cel, u, G);
+    __syncthreads();   // B's reads
+    // S_im = sum_kn C^{ik}_mn G_kn.  The record holds C^{ik} of the six pairs i <= k (0,0 1,1 2,2 0,1
+    // 0,2 1,2); C^{ki}_mn = C^{ik}_nm.
+    const double *rec = qp + e * (int64_t)QS * Q3 + (int64_t)Q_D * Q3 + g;
+    const auto field = [&](int f) -> double {
+        if constexpr (CK == 1) return (double)cr[f];
+        else if constexpr (CK == 2) return (double)__uint_as_float(f & 1 ? cw[f >> 1] & 0xFFFF0000u : cw[f >> 1] << 16);
+        else return rec[(int64_t)f * Q3];
+    };
 #pragma unroll
-        for (int ab = 0; ab < P1; ++ab) xv[ab] = sA[k * N3 + ab * PP + r];
-        double *o = sB + kb * Q * PP + r;
+    for (int q = 0; q < 9; ++q) S[q] = 0.0;
 #pragma unroll
-        for (int qb = 0; qb < Q; ++qb) {
-            double s = 0.0;
+    for (int p = 0; p < 6; ++p) {
+        const int i = p < 3 ? p : (p == 5 ? 1 : 0), k = p < 3 ? p : (p == 3 ? 1 : 2);
+        double cv[9];
 #pragma unroll
-            for (int ab = 0; ab < P1; ++ab) s += sF[2][sb][ab][qb] * xv[ab];
-            o[qb * PP] = s;
+        for (int mn = 0; mn < 9; ++mn) cv[mn] = field(9 * p + mn);
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+            S[3 * m + i] += cv[3 * m] * G[k] + cv[3 * m + 1] * G[3 + k] + cv[3 * m + 2] * G[6 + k];
+        if (i != k) {
+#pragma unroll
+            for (int m = 0; m < 3; ++m) S[3 * m + k] += cv[m] * G[i] + cv[3 + m] * G[3 + i] + cv[6 + m] * G[6 + i];
         }
     }
+    if (valid) c.put_point(pel, C::point(u), S);
     __syncthreads();
-    // eta: U2 -> A, pencils (k n, qb, az)
-    for (int t = tid; t < 9 * Q * P1; t += NT) {
-        const int az = t % P1, qb = (t / P1) % Q, kn = t / (P1 * Q);
-        const int k = kn / 3, n = kn - 3 * k;
-        const int sb = n == 2, se = n == 1;
-        const double *u = sB + ((k * 2 + sb) * Q + qb) * PP + az;
-        double uv[P1];
-#pragma unroll
-        for (int ae = 0; ae < P1; ++ae) uv[ae] = u[ae * P1];
-        double *o = sA + (kn * Q + qb) * Q * P1 + az;
-#pragma unroll
-        for (int qe = 0; qe < Q; ++qe) {
-            double s = 0.0;
-#pragma unroll
-            for (int ae = 0; ae < P1; ++ae) s += sF[1][se][ae][qe] * uv[ae];
-            o[qe * P1] = s;
-        }
-    }
-    __syncthreads();
-    // zeta: G -> B, pencils (k n, qb qe)
-    for (int t = tid; t < 9 * QQ; t += NT) {
-        const int qbe = t % QQ, kn = t / QQ;
-        const int n = kn % 3;
-        const double *u = sA + (kn * QQ + qbe) * P1;
-        double uv[P1];
-#pragma unroll
-        for (int az = 0; az < P1; ++az) uv[az] = u[az];
-        double *o = sB + kn * Q3 + qbe * Q;
-#pragma unroll
-        for (int qz = 0; qz < Q; ++qz) {
-            double s = 0.0;
-#pragma unroll
-            for (int az = 0; az < P1; ++az) s += sF[0][n == 0][az][qz] * uv[az];
-            o[qz] = s;
-        }
-    }
-    __syncthreads();
-    // per point: S_im = sum_kn C^{ik}_mn G_kn, in place in B.  The record holds C^{ik} of the six
-    // pairs i <= k (0,0 1,1 2,2 0,1 0,2 1,2); C^{ki}_mn = C^{ik}_nm.
-    const double *rec = qp + e * (int64_t)QS * Q3 + (int64_t)Q_D * Q3;
-    for (int g = tid; g < Q3; g += NT) {
-        const int t = min(max((int)sT[g], 0), Q3 - 1);
-        double gk[3][3], S[3][3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-#pragma unroll
-            for (int n = 0; n < 3; ++n) {
-                gk[k][n] = sB[(3 * k + n) * Q3 + t];
-                S[k][n] = 0.0;
-            }
-#pragma unroll
-        for (int p = 0; p < 6; ++p) {
-            const int i = p < 3 ? p : (p == 5 ? 1 : 0), k = p < 3 ? p : (p == 3 ? 1 : 2);
-            double c[9];
-#pragma unroll
-            for (int mn = 0; mn < 9; ++mn) {
-                if constexpr (C32)
-                    c[mn] = (double)cr[9 * p + mn];
-                else
-                    c[mn] = rec[(int64_t)(9 * p + mn) * Q3 + g];
-            }
-#pragma unroll
-            for (int m = 0; m < 3; ++m)
-                S[i][m] += c[3 * m] * gk[k][0] + c[3 * m + 1] * gk[k][1] + c[3 * m + 2] * gk[k][2];
-            if (i != k) {
-#pragma unroll
-                for (int m = 0; m < 3; ++m) S[k][m] += c[m] * gk[i][0] + c[3 + m] * gk[i][1] + c[6 + m] * gk[i][2];
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-            for (int m = 0; m < 3; ++m) sB[(3 * i + m) * Q3 + t] = S[i][m];
-    }
-    __syncthreads();
-    // zeta transposed: W -> A, pencils (i m, qb qe)
-    for (int t = tid; t < 9 * QQ; t += NT) {
-        const int qbe = t % QQ, im = t / QQ;
-        const int m = im % 3;
-        const double *sv = sB + im * Q3 + qbe * Q;
-        double v[Q];
-#pragma unroll
-        for (int qz = 0; qz < Q; ++qz) v[qz] = sv[qz];
-        double *o = sA + (im * QQ + qbe) * P1;
-#pragma unroll
-        for (int az = 0; az < P1; ++az) {
-            double s = 0.0;
-#pragma unroll
-            for (int qz = 0; qz < Q; ++qz) s += sF[0][m == 0][az][qz] * v[qz];
-            o[az] = s;
-        }
-    }
-    __syncthreads();
-    // eta transposed: Z -> B, pencils (i, sb, qb, az)
-    for (int t = tid; t < 6 * Q * P1; t += NT) {
-        const int az = t % P1, qb = (t / P1) % Q, is = t / (P1 * Q);
-        const int i = is >> 1, sb = is & 1;
-        double *o = sB + ((i * 2 + sb) * Q + qb) * PP + az;
-        if (sb == 0) {
-            const double *w0 = sA + ((i * 3) * QQ + qb * Q) * P1 + az;
-            const double *w1 = sA + ((i * 3 + 1) * QQ + qb * Q) * P1 + az;
-            double a0[Q], a1[Q];
-#pragma unroll
-            for (int qe = 0; qe < Q; ++qe) {
-                a0[qe] = w0[qe * P1];
-                a1[qe] = w1[qe * P1];
-            }
-#pragma unroll
-            for (int ae = 0; ae < P1; ++ae) {
-                double s = 0.0;
-#pragma unroll
-                for (int qe = 0; qe < Q; ++qe) s += sF[1][0][ae][qe] * a0[qe] + sF[1][1][ae][qe] * a1[qe];
-                o[ae * P1] = s;
-            }
-        } else {
-            const double *w2 = sA + ((i * 3 + 2) * QQ + qb * Q) * P1 + az;
-            double a2[Q];
-#pragma unroll
-            for (int qe = 0; qe < Q; ++qe) a2[qe] = w2[qe * P1];
-#pragma unroll
-            for (int ae = 0; ae < P1; ++ae) {
-                double s = 0.0;
-#pragma unroll
-                for (int qe = 0; qe < Q; ++qe) s += sF[1][0][ae][qe] * a2[qe];
-                o[ae * P1] = s;
-            }
-        }
-    }
-    __syncthreads();
-    // beta transposed: y, in local node order, pencils (i, ae az)
-    double *yo = ye + e * (int64_t)N3 * 3;
-    for (int t = tid; t < 3 * PP; t += NT) {
-        const int r = t % PP, i = t / PP;
-        double z0[Q], z1[Q];
-#pragma unroll
-        for (int qb = 0; qb < Q; ++qb) {
-            z0[qb] = sB[((i * 2) * Q + qb) * PP + r];
-            z1[qb] = sB[((i * 2 + 1) * Q + qb) * PP + r];
-        }
-#pragma unroll
-        for (int ab = 0; ab < P1; ++ab) {
-            double s = 0.0;
-#pragma unroll
-            for (int qb = 0; qb < Q; ++qb) s += sF[2][0][ab][qb] * z0[qb] + sF[2][1][ab][qb] * z1[qb];
-            yo[3 * sLoc[ab * PP + r] + i] = s;
-        }
-    }
+    c.to_nodes(e0, ye, elements, nullptr, nullptr);
 }
 
 // c32[e][f][g] = (float) records' C field f at point g (f < 54)

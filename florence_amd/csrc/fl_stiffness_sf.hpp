@@ -56,27 +56,259 @@ __device__ __forceinline__ void traction_point_tensor(const double *ix, const do
         for (int i = 0; i < 3; ++i) P[3 * m + i] = ix[m] * Si[i][0] + ix[3 + m] * Si[i][1] + ix[6 + m] * Si[i][2];
 }
 
-// Phase 1 for tensor-product hexes: a workgroup of 128 threads (256 for 6^3 points) for the
-// EPB elements whose points fill it, a point per thread.  The elements' X and x are staged in LDS in tensor
-// node order and the parent Jacobians at all points, dX_c/dxi_m = sum_a dN_a/dxi_m X_a,c,
-// are contracted one direction at a time:
+// The sum factorisation of a point kernel, shared by qp_sf_kernel (X and x, NF = 6) and
+// mf_element_kernel (a dof vector, NF = 3): a workgroup of 128 threads (256 for 6^3 points)
+// for the EPB elements whose points fill it, a point per thread.  Gradients of the NF
+// fields at all points, one direction at a time:
 //
 //     A[f][s0][ab,ae][qz]   = sum_az T0^{s0}[az][qz] X_f[ab,ae,az]
 //     B[f][m][ab][qe,qz]    = sum_ae T1^{[m=1]}[ae][qe] A[f][[m=0]][ab,ae][qz]
 //     P[f][m][qb,qe,qz]     = sum_ab T2^{[m=2]}[ab][qb] B[f][m][ab][qe,qz]
 //
-// (f = X_0..2, x_0..2: A for all six, then B and P for X and for x), then each point runs
-// qp_point.  Same records as qp_kernel, to rounding (the node sum is taken in another
-// order).  With te given, the element tractions
-// t_(a,i) = sum_q sum_m dN_a/dxi_m (q) P[q][m][i] follow in the same workgroup: the point
-// tensors contracted zeta, eta, beta in turn for the nine (m, i); the records -- if qp is
-// given at all -- then omit detJ sigma and detJ.  te in local node order; with T, a node of
-// one element only gets its T entry directly (as 0.0 + value, the accumulated form).
+// (B and P for three fields at a time), and back from point tensors P[q][m][i] to nodes,
+// t_(a,i) = sum_q sum_m dN_a/dxi_m (q) P[q][m][i], contracted zeta, eta, beta in turn.
 //
 // A task is a line: a thread reads the line's values once, forms every output of the
 // contraction with them in registers and takes the 1D basis, the same for a whole wave,
 // from scalar registers; only P's basis depends on the thread's point.  LDS strides are odd
-// where the lanes of an access step over a line.  Bound by VALU issue and LDS together
+// where the lanes of an access step over a line.
+typedef const double __attribute__((address_space(4))) ConstDouble;
+
+template <int P1, int Q, int NF>
+struct SfLines {
+    typedef SfLayout<P1, Q> L;
+    static constexpr int Q3 = L::Q3, N3 = L::N3, PP = L::PP, QQ = Q * Q;
+    static constexpr int NT = Q3 <= 128 ? 128 : 256, EPB = NT / Q3, NW = NT / 64;
+    static constexpr int XS = P1 | 1, AS = Q | 1, PS = QQ | 1;   // line strides in LDS
+    static constexpr int NWB = (EPB * 3 * P1 * Q + 63) / 64;     // waves' worth of B lines of a kind
+    static constexpr int KB = (2 * NWB + NW - 1) / NW;           // of them, a wave's
+    // three fields: B is written over A once every line is read, X staged in the space above A
+    static constexpr bool ONE = NF == 3;
+    static constexpr int SZ_X = NF * PP * XS, SZ_B = 9 * P1 * QQ, SZ_A = 2 * NF * PP * AS;
+    static constexpr int SZ_P = 9 * Q * PS;   // the point tensors, then U1 and U2 in place
+    static constexpr int mx(int a, int b) { return a > b ? a : b; }
+    static constexpr int SZ_AP = ONE ? mx(SZ_A + SZ_X, mx(SZ_B, SZ_P)) : mx(SZ_A, SZ_P);
+    static constexpr int SZ_XB = ONE ? SZ_AP : mx(SZ_X, SZ_B);
+    static constexpr int X0 = ONE ? SZ_A : 0;
+    // which waves take a stage's tasks first, so that the stages whose tasks do not fill the
+    // workgroup evenly (A, the last few of U1 and U2, t) and B's two weights add up evenly
+    static constexpr int ROT_A = NW / 2, ROT_U = NF == 3 ? NW / 2 : 0, ROT_T = NF == 3 ? 0 : NW / 2;
+    static constexpr int LDS = EPB * (SZ_AP + (ONE ? 0 : SZ_XB));
+    static_assert(EPB >= 1, "one point per thread");
+
+    const double *f1d;
+    const int32_t *loc;   // local node of tensor node
+    int ne, tid, wave, lane;
+    double *sXB, *sAP;
+
+    // the 1D basis s (0 values, 1 derivatives) of direction d, read through scalar loads where
+    // it is used: an address the compiler cannot trace keeps it from holding all of them in
+    // registers over the whole kernel
+    __device__ __forceinline__ ConstDouble *f(int d, int s) const {
+        uint64_t a = reinterpret_cast<uint64_t>(f1d + (d * 2 + s) * P1 * Q);
+        asm volatile("" : "+s"(a));
+        return reinterpret_cast<ConstDouble *>(a);
+    }
+    // where field f's value at tensor node tn of element el is staged
+    __device__ __forceinline__ double *x(int el, int fi, int tn) const {
+        return sXB + el * SZ_XB + X0 + (fi * PP + tn / P1) * XS + tn % P1;
+    }
+    // A: line (element, f, ab, ae)
+    __device__ __forceinline__ void form_A() const {
+        for (int t = tid ^ (ROT_A * 64); t < ne * NF * PP; t += NT) {
+            const int el = EPB == 1 ? 0 : t / (NF * PP), r = t - el * NF * PP, fi = r / PP, abe = r - fi * PP;
+            const double *x = sXB + el * SZ_XB + X0 + r * XS;
+            double v[P1];
+#pragma unroll
+            for (int az = 0; az < P1; ++az) v[az] = x[az];
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                double *a = sAP + el * SZ_AP + ((fi * 2 + s) * PP + abe) * AS;
+                ConstDouble *l = f(0, s);
+#pragma unroll
+                for (int qz = 0; qz < Q; ++qz) {
+                    double acc = 0.0;
+#pragma unroll
+                    for (int az = 0; az < P1; ++az) acc += l[az * Q + qz] * v[az];
+                    a[qz] = acc;
+                }
+            }
+        }
+    }
+    // B of fields f0 .. f0 + 2: line (element, f, ab, qz), those of A's s0 = 0 giving m = 1 and
+    // 2, those of s0 = 1 giving m = 0; a wave's lines are of one kind
+    __device__ __forceinline__ void form_B(int f0) const {
+        double v[KB][P1];
+        double *bo[KB];
+        const auto read = [&](int j) {
+            const int wt = wave + j * NW, s0 = wt >= NWB;
+            const int t = (wt - s0 * NWB) * 64 + lane;
+            const bool on = wt < 2 * NWB && t < ne * 3 * P1 * Q;
+            const int tc = on ? t : 0;
+            const int el = EPB == 1 ? 0 : tc / (3 * P1 * Q), r = tc - el * 3 * P1 * Q;
+            const int fi = r / (P1 * Q), ab = (r / Q) % P1, qz = r % Q;
+            const double *a = sAP + el * SZ_AP + (((f0 + fi) * 2 + s0) * PP + ab * P1) * AS + qz;
+            bo[j] = on ? sXB + el * SZ_XB + (fi * 3 * P1 + ab) * QQ + qz : nullptr;
+#pragma unroll
+            for (int ae = 0; ae < P1; ++ae) v[j][ae] = a[ae * AS];
+        };
+        const auto write = [&](int j) {
+            const auto contract = [&](int m) {
+                ConstDouble *l = f(1, m == 1);
+#pragma unroll
+                for (int qe = 0; qe < Q; ++qe) {
+                    double acc = 0.0;
+#pragma unroll
+                    for (int ae = 0; ae < P1; ++ae) acc += l[ae * Q + qe] * v[j][ae];
+                    if (bo[j]) bo[j][m * P1 * QQ + qe * Q] = acc;
+                }
+            };
+            if (wave + j * NW >= NWB) {
+                contract(0);
+            } else {
+                contract(1);
+                contract(2);
+            }
+        };
+        if constexpr (ONE) {
+#pragma unroll
+            for (int j = 0; j < KB; ++j) read(j);
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < KB; ++j)
+                if (wave + j * NW < 2 * NWB) write(j);
+        } else {
+#pragma unroll
+            for (int j = 0; j < KB; ++j)
+                if (wave + j * NW < 2 * NWB) {
+                    read(j);
+                    write(j);
+                }
+        }
+    }
+    // tensor point of thread u of an element, beta fastest: the order of the quadrature rules,
+    // so that a wave's record accesses are contiguous (the record point is the basis table's)
+    static __device__ __forceinline__ int point(int u) { return (u % Q * Q + u / Q % Q) * Q + u / QQ; }
+    // P[3 m + c] of B's three fields at the point of thread u of element el; sFb: the beta basis
+    __device__ __forceinline__ void gradient(const double (&sFb)[2][P1][Q], int el, int u, double (&P)[9]) const {
+        const int qb = u % Q, qe = u / Q % Q, qz = u / QQ;
+        const double *bb = sXB + el * SZ_XB + qe * Q + qz;
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                double acc = 0.0;
+#pragma unroll
+                for (int ab = 0; ab < P1; ++ab) acc += sFb[m == 2][ab][qb] * bb[((c * 3 + m) * P1 + ab) * QQ];
+                asm volatile("" : "+v"(acc));   // summed here: its operands are not kept for later
+                P[3 * m + c] = acc;
+            }
+    }
+    // the point tensor P[3 m + i] at tensor point tq of element el, for to_nodes
+    __device__ __forceinline__ void put_point(int el, int tq, const double (&P)[9]) const {
+        double *po = sAP + el * SZ_AP + (tq % Q) * PS + (tq / Q) % Q * Q + tq / QQ;
+#pragma unroll
+        for (int mi = 0; mi < 9; ++mi) po[mi * Q * PS] = P[mi];
+    }
+    // lines of the nine (m, i), those whose m takes the derivatives of direction D (m == D)
+    // first; a wave's lines are of one kind: task(el, mi, r, basis) of r in [0, R)
+    template <int D, int R, typename Task>
+    __device__ __forceinline__ void lines(const Task &task) const {
+        constexpr int n1 = (EPB * 3 * R + 63) / 64, n2 = (EPB * 6 * R + 63) / 64;
+        for (int wt = wave ^ ROT_U; wt < n1 + n2; wt += NW) {
+            if (wt < n1) {
+                const int t = wt * 64 + lane;
+                if (t < ne * 3 * R) {
+                    const int el = EPB == 1 ? 0 : t / (3 * R), r = t - el * 3 * R, j = r / R;
+                    task(el, 3 * D + j, r - j * R, f(D, 1));
+                }
+            } else {
+                const int t = (wt - n1) * 64 + lane;
+                if (t < ne * 6 * R) {
+                    const int el = EPB == 1 ? 0 : t / (6 * R), r = t - el * 6 * R, j = r / R;
+                    // m = 1, 2 (D = 0) or 0, 2 (D = 1)
+                    task(el, D == 0 || j >= 3 ? 3 + j : j, r - j * R, f(D, 0));
+                }
+            }
+        }
+    }
+    // after a barrier that follows put_point: the node vectors of elements e0 .. e0 + ne - 1
+    // to te [e][local node][3]; with T, a node of one element only gets its T entry directly
+    // (as 0.0 + value, the accumulated form)
+    __device__ __forceinline__ void to_nodes(int64_t e0, double *__restrict__ te,
+                                             const int32_t *__restrict__ elements,
+                                             const int32_t *__restrict__ node_elem_ptr,
+                                             double *__restrict__ T) const {
+        // a line's outputs go where its inputs were: U1 [mi][az][qe, qb] in P [mi][qz][qe, qb]
+        lines<0, QQ>([&](int el, int mi, int r, ConstDouble *l) {
+            double *p = sAP + el * SZ_AP + mi * Q * PS + r;
+            double v[Q];
+#pragma unroll
+            for (int qz = 0; qz < Q; ++qz) v[qz] = p[qz * PS];
+#pragma unroll
+            for (int az = 0; az < P1; ++az) {
+                double acc = 0.0;
+#pragma unroll
+                for (int qz = 0; qz < Q; ++qz) acc += l[az * Q + qz] * v[qz];
+                p[az * PS] = acc;
+            }
+        });
+        __syncthreads();
+        // U2 [mi][az][ae, qb] in U1
+        lines<1, P1 * Q>([&](int el, int mi, int r, ConstDouble *l) {
+            const int az = r / Q;
+            double *p = sAP + el * SZ_AP + (mi * Q + az) * PS + r - az * Q;
+            double v[Q];
+#pragma unroll
+            for (int qe = 0; qe < Q; ++qe) v[qe] = p[qe * Q];
+#pragma unroll
+            for (int ae = 0; ae < P1; ++ae) {
+                double acc = 0.0;
+#pragma unroll
+                for (int qe = 0; qe < Q; ++qe) acc += l[ae * Q + qe] * v[qe];
+                p[ae * Q] = acc;
+            }
+        });
+        __syncthreads();
+        for (int t = tid ^ (ROT_T * 64); t < ne * 3 * PP; t += NT) {
+            const int el = EPB == 1 ? 0 : t / (3 * PP), r = t - el * 3 * PP, aeaz = r / 3, i = r - 3 * aeaz;
+            double s[P1];
+#pragma unroll
+            for (int ab = 0; ab < P1; ++ab) s[ab] = 0.0;
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                const double *u = sAP + el * SZ_AP + ((3 * m + i) * Q + aeaz % P1) * PS + aeaz / P1 * Q;
+                ConstDouble *l = f(2, m == 2);
+                double v[Q];
+#pragma unroll
+                for (int q = 0; q < Q; ++q) v[q] = u[q];
+#pragma unroll
+                for (int ab = 0; ab < P1; ++ab)
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) s[ab] += l[ab * Q + q] * v[q];
+            }
+            const int64_t ee = e0 + el;
+#pragma unroll
+            for (int ab = 0; ab < P1; ++ab) {
+                const int lt = min(max(loc[ab * PP + aeaz], 0), N3 - 1);
+                te[ee * 3 * N3 + 3 * lt + i] = s[ab];
+                if (T) {
+                    const int32_t a = elements[ee * N3 + lt];
+                    if (node_elem_ptr[a + 1] - node_elem_ptr[a] == 1) T[3 * (int64_t)a + i] = 0.0 + s[ab];
+                }
+            }
+        }
+    }
+};
+
+// Phase 1 for tensor-product hexes, with SfLines: the elements' X and x are staged in LDS in
+// tensor node order and the parent Jacobians at all points, dX_c/dxi_m = sum_a dN_a/dxi_m
+// X_a,c, are contracted one direction at a time; then each point runs qp_point.  Same records
+// as qp_kernel, to rounding (the node sum is taken in another order).  With te given, the
+// element tractions follow in the same workgroup from the point tensors; the records -- if qp
+// is given at all -- then omit detJ sigma and detJ.
+//
+// Bound by VALU issue and LDS together
 // (p = 4, 6^3 points: 1004 VALU and 163 LDS instructions a wave, half the cycles each); a
 // task an output, which reads both factors of every product from LDS, and a workgroup an
 // element at every p were LDS-bound, and idle at small p.  Residual pass before -> now: p = 4,
@@ -84,22 +316,8 @@ __device__ __forceinline__ void traction_point_tensor(const double *ix, const do
 // the assembly: 352 -> 230, 182 -> 68, 77 -> 26.  A thread takes record point g, not tensor
 // point g: its wave's 54 record stores are then contiguous (p = 4, 20^3 284 -> 230).  Two points a thread, for half of P's reads,
 // do not pay (134, and 617 for the tangent, whose registers then spill).
-typedef const double __attribute__((address_space(4))) ConstDouble;
-
-template <int P1, int Q>
-struct QpSf {
-    typedef SfLayout<P1, Q> L;
-    static constexpr int NT = L::Q3 <= 128 ? 128 : 256, QQ = Q * Q, EPB = NT / L::Q3;
-    static constexpr int XS = P1 | 1, AS = Q | 1, PS = QQ | 1;   // line strides in LDS
-    static constexpr int SZ_X = 6 * L::PP * XS, SZ_B = 9 * P1 * QQ;          // U1 [9][P1][QQ] in B's space
-    static constexpr int SZ_A = 12 * L::PP * AS, SZ_P = 9 * Q * PS;          // U2 [9][PP][AS] in A's space
-    static constexpr int SZ_XB = SZ_X > SZ_B ? SZ_X : SZ_B, SZ_AP = SZ_A > SZ_P ? SZ_A : SZ_P;
-    static_assert(EPB >= 1, "one point per thread");
-    static_assert(9 * L::PP * AS <= SZ_AP, "U2 in A's space");
-};
-
 template <int P1, int Q, bool TANGENT, bool GEN>
-__global__ __launch_bounds__((QpSf<P1, Q>::NT), TANGENT ? (GEN ? 2 : 3) : 4) void qp_sf_kernel(MatParams mp0, const double *__restrict__ points,
+__global__ __launch_bounds__((SfLines<P1, Q, 6>::NT), TANGENT ? (GEN ? 2 : 3) : 4) void qp_sf_kernel(MatParams mp0, const double *__restrict__ points,
                                                     const int32_t *__restrict__ elements,
                                                     const double *__restrict__ Eulerx,
                                                     const int32_t *__restrict__ basis, const double *__restrict__ w,
@@ -109,214 +327,61 @@ __global__ __launch_bounds__((QpSf<P1, Q>::NT), TANGENT ? (GEN ? 2 : 3) : 4) voi
                                                     double *__restrict__ te = nullptr,
                                                     const int32_t *__restrict__ node_elem_ptr = nullptr,
                                                     double *__restrict__ T = nullptr) {
-    typedef SfLayout<P1, Q> L;
-    typedef QpSf<P1, Q> C;
-    constexpr int Q3 = L::Q3, N3 = L::N3, PP = L::PP, QQ = C::QQ, EPB = C::EPB, NT = C::NT;
-    constexpr int XS = C::XS, AS = C::AS, PS = C::PS, SZ_XB = C::SZ_XB, SZ_AP = C::SZ_AP;
+    typedef SfLines<P1, Q, 6> C;
+    constexpr int Q3 = C::Q3, N3 = C::N3, EPB = C::EPB, NT = C::NT;
     __shared__ double sFb[2][P1][Q];
-    __shared__ double sXB[EPB * SZ_XB];
-    __shared__ double sAP[EPB * SZ_AP];
-    __shared__ int16_t sTg[Q3];   // tensor point of record point g
+    __shared__ double sAP[C::LDS];
+    double *sXB = sAP + EPB * C::SZ_AP;
     const int64_t e0 = (int64_t)blockIdx.x * EPB;
     const int ne = (int)min((int64_t)EPB, nelem - e0);
     if (ne <= 0) return;
     const int tid = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int32_t *g_of_t = basis + 4;
     const int32_t *loc = basis + 4 + Q3;
-    const double *f1d = reinterpret_cast<const double *>(basis + L::INTS);
-    // 1D basis s (0 values, 1 derivatives) of direction d, read through scalar loads where it
-    // is used: an address the compiler cannot trace keeps it from holding all of them in
-    // registers over the whole kernel
-    const auto f = [&](int d, int s) {
-        uint64_t a = reinterpret_cast<uint64_t>(f1d + (d * 2 + s) * P1 * Q);
-        asm volatile("" : "+s"(a));
-        return reinterpret_cast<const ConstDouble *>(a);
-    };
+    const double *f1d = reinterpret_cast<const double *>(basis + SfLayout<P1, Q>::INTS);
+    const C c = {f1d, loc, ne, tid, __builtin_amdgcn_readfirstlane(tid >> 6), tid & 63, sXB, sAP};
     for (int t = tid; t < 2 * P1 * Q; t += NT) (&sFb[0][0][0])[t] = f1d[4 * P1 * Q + t];
     // table entries are clamped into range
-    for (int t = tid; t < Q3; t += NT) sTg[min(max(g_of_t[t], 0), Q3 - 1)] = (int16_t)t;
     for (int t = tid; t < ne * N3; t += NT) {
-        const int el = t / N3, tn = t - el * N3;
+        const int el = EPB == 1 ? 0 : t / N3, tn = t - el * N3;
         const int64_t nd = elements[(e0 + el) * N3 + min(max(loc[tn], 0), N3 - 1)];
-        double *x = sXB + el * SZ_XB + (tn / P1) * XS + tn % P1;
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            x[c * PP * XS] = points[3 * nd + c];
-            x[(3 + c) * PP * XS] = Eulerx[3 * nd + c];
+        for (int k = 0; k < 3; ++k) {
+            *c.x(el, k, tn) = points[3 * nd + k];
+            *c.x(el, 3 + k, tn) = Eulerx[3 * nd + k];
         }
     }
     __syncthreads();
-    // A: line (element, f, ab, ae)
-    for (int t = tid; t < ne * 6 * PP; t += NT) {
-        const int el = t / (6 * PP), r = t - el * 6 * PP, fi = r / PP, abe = r - fi * PP;
-        const double *x = sXB + el * SZ_XB + r * XS;
-        double v[P1];
-#pragma unroll
-        for (int az = 0; az < P1; ++az) v[az] = x[az];
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            double *a = sAP + el * SZ_AP + ((fi * 2 + s) * PP + abe) * AS;
-            const ConstDouble *l = f(0, s);
-#pragma unroll
-            for (int qz = 0; qz < Q; ++qz) {
-                double acc = 0.0;
-#pragma unroll
-                for (int az = 0; az < P1; ++az) acc += l[az * Q + qz] * v[az];
-                a[qz] = acc;
-            }
-        }
-    }
-    // this thread's point: record point g, so that a wave's record stores are contiguous
-    const int pel = tid / Q3, g = tid - pel * Q3;
+    c.form_A();
+    const int pel = tid / Q3, tq = C::point(tid - pel * Q3);
     const bool valid = pel < ne;
     const int cel = valid ? pel : 0;
-    const int tq = min(max((int)sTg[g], 0), Q3 - 1);
-    const int qb = tq / QQ, qez = tq - qb * QQ;
     double PJ[2][9];
 #pragma unroll
     for (int pass = 0; pass < 2; ++pass) {
         __syncthreads();   // A written; the previous pass's reads of B done
-        // B: lines (element, f, ab, qz), those of A's s0 = 0 giving m = 1 and 2, those of
-        // s0 = 1 giving m = 0; a wave's lines are of one kind
-        constexpr int NW = (EPB * 3 * P1 * Q + 63) / 64;
-        for (int wt = wave; wt < 2 * NW; wt += NT / 64) {
-            const int s0 = wt >= NW;
-            const int t = (wt - s0 * NW) * 64 + lane;
-            if (t < ne * 3 * P1 * Q) {
-                const int el = t / (3 * P1 * Q), r = t - el * 3 * P1 * Q;
-                const int fi = r / (P1 * Q), ab = (r / Q) % P1, qz = r % Q;
-                const double *a = sAP + el * SZ_AP + (((3 * pass + fi) * 2 + s0) * PP + ab * P1) * AS + qz;
-                double *bo = sXB + el * SZ_XB + (fi * 3 * P1 + ab) * QQ + qz;
-                double v[P1];
-#pragma unroll
-                for (int ae = 0; ae < P1; ++ae) v[ae] = a[ae * AS];
-                const auto contract = [&](int m) {
-                    const ConstDouble *l = f(1, m == 1);
-#pragma unroll
-                    for (int qe = 0; qe < Q; ++qe) {
-                        double acc = 0.0;
-#pragma unroll
-                        for (int ae = 0; ae < P1; ++ae) acc += l[ae * Q + qe] * v[ae];
-                        bo[m * P1 * QQ + qe * Q] = acc;
-                    }
-                };
-                if (s0) {
-                    contract(0);
-                } else {
-                    contract(1);
-                    contract(2);
-                }
-            }
-        }
+        c.form_B(3 * pass);
         __syncthreads();
-        // P at this thread's point
-        const double *bb = sXB + cel * SZ_XB + qez;
-#pragma unroll
-        for (int m = 0; m < 3; ++m)
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                double acc = 0.0;
-#pragma unroll
-                for (int ab = 0; ab < P1; ++ab) acc += sFb[m == 2][ab][qb] * bb[((c * 3 + m) * P1 + ab) * QQ];
-                asm volatile("" : "+v"(acc));   // summed here: its operands are not kept for later
-                PJ[pass][3 * m + c] = acc;
-            }
+        c.gradient(sFb, cel, tid - pel * Q3, PJ[pass]);
     }
+    const int g = min(max(g_of_t[tq], 0), Q3 - 1);
     const int64_t e = e0 + cel;
     const MatParams mp = element_material(mp0, e, elem_mat, mat_table);
     // te given: the element tractions are contracted here from the point values, and
     // the records (qp, when given) are only what the stiffness kernels read
     double pv[15];
     qp_point<TANGENT, GEN>(mp, PJ[0], PJ[1], w[g], update, valid,
-                      qp ? qp + e * (int64_t)Q3 * (TANGENT ? QS : QS_RES) + g : nullptr, Q3, status, emitC != 0,
-                      te != nullptr, pv);
+                           qp ? qp + e * (int64_t)Q3 * (TANGENT ? QS : QS_RES) + g : nullptr, Q3, status,
+                           emitC != 0, te != nullptr, pv);
     if (!te) return;
     // A's last reads precede the barrier before the second P
     if (valid) {
         double P[9];
         traction_point_tensor(pv, pv + 9, P);
-        double *po = sAP + pel * SZ_AP + (tq % Q) * PS + (tq / Q) % Q * Q + qb;
-#pragma unroll
-        for (int mi = 0; mi < 9; ++mi) po[mi * Q * PS] = P[mi];
+        c.put_point(pel, tq, P);
     }
     __syncthreads();
-    // lines of the nine (m, i), those whose m takes the derivatives of direction D (m == D)
-    // first; a wave's lines are of one kind: task(el, mi, r, basis) of r in [0, R)
-    const auto lines = [&](int D, int R, const auto &task) {
-        const int n1 = (EPB * 3 * R + 63) / 64, n2 = (EPB * 6 * R + 63) / 64;
-        for (int wt = wave; wt < n1 + n2; wt += NT / 64) {
-            const int s = wt < n1, k = s ? 3 : 6;
-            const int t = (s ? wt : wt - n1) * 64 + lane;
-            if (t < ne * k * R) {
-                const int el = t / (k * R), r2 = t - el * k * R, j = r2 / R;
-                // m of the others: 1, 2 (D = 0) or 0, 2 (D = 1)
-                const int m = s ? D : (j < 3 ? 1 - D : 2);
-                task(el, 3 * m + j % 3, r2 - j * R, f(D, s));
-            }
-        }
-    };
-    // U1 [mi][az][qe, qb]
-    lines(0, QQ, [&](int el, int mi, int r, const ConstDouble *l) {
-        const double *p = sAP + el * SZ_AP + mi * Q * PS + r;
-        double *u = sXB + el * SZ_XB + mi * P1 * QQ + r;
-        double v[Q];
-#pragma unroll
-        for (int qz = 0; qz < Q; ++qz) v[qz] = p[qz * PS];
-#pragma unroll
-        for (int az = 0; az < P1; ++az) {
-            double acc = 0.0;
-#pragma unroll
-            for (int qz = 0; qz < Q; ++qz) acc += l[az * Q + qz] * v[qz];
-            u[az * QQ] = acc;
-        }
-    });
-    __syncthreads();
-    // U2 [mi][ae, az][qb]
-    lines(1, P1 * Q, [&](int el, int mi, int r, const ConstDouble *l) {
-        const int az = r / Q, q = r - az * Q;
-        const double *p = sXB + el * SZ_XB + (mi * P1 + az) * QQ + q;
-        double *u = sAP + el * SZ_AP + (mi * PP + az) * AS + q;
-        double v[Q];
-#pragma unroll
-        for (int qe = 0; qe < Q; ++qe) v[qe] = p[qe * Q];
-#pragma unroll
-        for (int ae = 0; ae < P1; ++ae) {
-            double acc = 0.0;
-#pragma unroll
-            for (int qe = 0; qe < Q; ++qe) acc += l[ae * Q + qe] * v[qe];
-            u[ae * P1 * AS] = acc;
-        }
-    });
-    __syncthreads();
-    for (int t = tid; t < ne * 3 * PP; t += NT) {
-        const int el = t / (3 * PP), r = t - el * 3 * PP, aeaz = r / 3, i = r - 3 * aeaz;
-        double s[P1];
-#pragma unroll
-        for (int ab = 0; ab < P1; ++ab) s[ab] = 0.0;
-#pragma unroll
-        for (int m = 0; m < 3; ++m) {
-            const double *u = sAP + el * SZ_AP + ((3 * m + i) * PP + aeaz) * AS;
-            const ConstDouble *l = f(2, m == 2);
-            double v[Q];
-#pragma unroll
-            for (int q = 0; q < Q; ++q) v[q] = u[q];
-#pragma unroll
-            for (int ab = 0; ab < P1; ++ab)
-#pragma unroll
-                for (int q = 0; q < Q; ++q) s[ab] += l[ab * Q + q] * v[q];
-        }
-        const int64_t ee = e0 + el;
-#pragma unroll
-        for (int ab = 0; ab < P1; ++ab) {
-            const int lt = min(max(loc[ab * PP + aeaz], 0), N3 - 1);
-            te[ee * 3 * N3 + 3 * lt + i] = s[ab];
-            if (T) {
-                const int32_t a = elements[ee * N3 + lt];
-                if (node_elem_ptr[a + 1] - node_elem_ptr[a] == 1) T[3 * (int64_t)a + i] = 0.0 + s[ab];
-            }
-        }
-    }
+    c.to_nodes(e0, te, elements, node_elem_ptr, T);
 }
 
 template <int P1, int Q>

@@ -248,6 +248,28 @@ def test_matrix_free_operator(cuda, case):
     assert np.array_equal(a, y2.cpu().numpy())
 
 
+@pytest.mark.parametrize("p,n", [(1, 1), (1, 3), (2, 1), (2, 3), (3, 3), (4, 1)])
+def test_matrix_free_element_groups(cuda, p, n):
+    """The element kernel takes 16, 4, 2 or 1 elements a workgroup and each XCD a range of
+    them: one element, and 27, which leaves workgroups in part or wholly empty.  The product
+    equals the CSR's to 1e-13."""
+    import torch
+    from florence_amd.assembly import DeviceMeshData, assemble_device
+    from florence_amd.materials import NeoHookean
+    from florence_amd.multigrid import mf_apply
+    from florence_amd.solver import spmv
+    m = cube_mesh("hex", p, n, jitter=0.05, seed=70 + p)
+    dm = DeviceMeshData(m, function_space(m, p))
+    V, _, _ = assemble_device(dm, NeoHookean(3, mu=1.0, lamb=10.0), deformed(m.points, 0.04, seed=71 + p))
+    free = torch.ones(3 * m.nnode, dtype=torch.uint8, device="cuda")
+    u = torch.as_tensor(np.sin(np.arange(3 * m.nnode) * 0.7), device="cuda")
+    y, z = torch.empty_like(u), torch.empty_like(u)
+    mf_apply(dm, free, u, y)
+    spmv(dm, V, u, z)
+    torch.cuda.synchronize()
+    assert float((y - z).abs().max() / z.abs().max()) <= 1e-13
+
+
 @pytest.mark.parametrize("precision", ["fp64", "fp32", "fp64-csr", "fp64-mf32", "fp64-mf64"])
 def test_multigrid_newton_matches_oracle(cuda, precision):
     """fp64: the default smoother (matrix-free from BF16 copies of the C values);
