@@ -427,6 +427,7 @@ __global__ __launch_bounds__(256) void qp_kernel(MatParams mp0, const double *__
 }  // namespace fl
 #include "fl_stiffness.hpp"
 #include "fl_stiffness_bf16.hpp"
+#include "fl_stiffness_el.hpp"
 #include "fl_stiffness_sf.hpp"
 #include "fl_stiffness_rows.hpp"
 #include "fl_mg_galerkin.hpp"
@@ -771,9 +772,36 @@ static int padded_np(int npe) {
     return -1;
 }
 
+// The element form of the dense FP64 contraction; false: not launched.  It takes the node
+// counts whose blocks are 16 x 16 tiles and at most four rows over, and rules whose points
+// fit 64 KB of LDS at once (two workgroups a CU: 79 points of 10 nodes, 64 of 20, 46 of 35);
+// 21 to 32 nodes and from 37 on would be padded as the pair form pads them.  A tile-shape
+// variant selected by FL_TUNE_STIFF_VARIANT_BASE is the pair form's.
+static bool launch_stiffness_el(int NP, const double *JmT, const double *qp, int npe, int G, int64_t nelem, double *Ke,
+                                hipStream_t st) {
+    if (nelem > INT32_MAX || (NP > 16 && tuning_value(TUNE_STIFF_VARIANT_BASE + NP / 16 - 1, 1) > 1)) return false;
+#define FL_EL_CASE(MT, REM, LO, HI)                                                                                 \
+    if (npe >= LO && npe <= HI && ElLayout<MT, REM>::lds(G) <= 64 * 1024) {                                          \
+        stiffness_el_kernel<MT, REM><<<(unsigned)nelem, 384, ElLayout<MT, REM>::lds(G), st>>>(JmT, NP, qp, npe, G,   \
+                                                                                             nelem, Ke);            \
+        return true;                                                                                                \
+    }
+    FL_EL_CASE(1, false, 1, 16)
+    FL_EL_CASE(1, true, 17, 20)
+    FL_EL_CASE(2, true, 33, 36)
+#undef FL_EL_CASE
+    return false;
+}
+
 template <typename CT, typename KT>
 static int launch_stiffness_t(int NP, const double *JmT, const double *qp, int npe, int G, int64_t nelem, KT *Ke,
                               hipStream_t st) {
+    if constexpr (sizeof(CT) == 8 && sizeof(KT) == 8) {
+        if (launch_stiffness_el(NP, JmT, qp, npe, G, nelem, Ke, st)) {
+            FL_LAUNCH_CHECK();
+            return 0;
+        }
+    }
     const int64_t groups = (nelem + 7) / 8 * 8 * 6;
     if (groups > (int64_t)INT32_MAX) {
         set_error("too many elements for one launch");

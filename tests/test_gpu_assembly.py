@@ -183,6 +183,24 @@ def test_dense_tile_variants(cuda, et, p, npc, variant):
         lib.fl_set_tuning(_lib.FL_TUNE_STIFF_SF, 0)
 
 
+@pytest.mark.parametrize("et,p,norder", [("tet", 1, 1), ("tet", 1, 5), ("tet", 2, 2), ("tet", 2, 3), ("tet", 3, 4),
+                                         ("tet", 3, 6), ("tet", 4, 6), ("hex", 1, 2), ("hex", 1, 4), ("hex", 1, 5)])
+def test_element_form_rules(cuda, et, p, norder):
+    """The element form of the dense contraction against the oracle: node counts that are a
+    part of a tile, a tile and four rows, two tiles and three rows; 3 G inner indices that
+    leave 0 to 3 of the last step; 1 point to 64, and 125, which the pair form takes."""
+    from florence_amd import _lib
+    lib = _lib.load()
+    _lib.check(lib.fl_set_tuning(_lib.FL_TUNE_STIFF_SF, 1), "fl_set_tuning")
+    try:
+        m = cube_mesh(et, p, 2 if p < 4 else 1, jitter=0.05, seed=21)
+        fs = function_space(m, p, norder=norder)
+        mat = MooneyRivlin(3, mu1=0.5, mu2=0.5, lamb=20.0)
+        _check(m, fs, mat, deformed(m.points, 0.04, seed=22), "{} p{} G={}".format(et, p, fs.AllGauss.shape[0]))
+    finally:
+        lib.fl_set_tuning(_lib.FL_TUNE_STIFF_SF, 0)
+
+
 @pytest.mark.parametrize("p", [1, 2, 3, 4])
 def test_sum_factorised_equals_dense(cuda, p):
     """Tensor-product hexes: the sum-factorised point, block and traction kernels (default
