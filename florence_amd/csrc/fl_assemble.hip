@@ -201,9 +201,12 @@ __global__ void zero_kernel(double *p, int64_t n) {
     if (i < n) p[i] = 0.0;
 }
 
-// Jm^T padded: JmT[(g*3+m)*NP + a] = dN_a/dxi_m at point g (0 for a >= npe)
-__global__ void transpose_jm_kernel(const double *__restrict__ Jm, int npe, int G, int NP, double *__restrict__ JmT) {
+// Jm^T padded: JmT[(g*3+m)*NP + a] = dN_a/dxi_m at point g (0 for a >= npe), and the status
+// cleared (a kernel, not a memset node, so the call can be graph-captured)
+__global__ void prepare_kernel(const double *__restrict__ Jm, int npe, int G, int NP, double *__restrict__ JmT,
+                               int32_t *__restrict__ status) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < 2) status[t] = 0;
     if (t >= G * 3 * NP) return;
     const int a = t % NP, m = (t / NP) % 3, g = t / (3 * NP);
     JmT[t] = a < npe ? Jm[((int64_t)m * npe + a) * G + g] : 0.0;
@@ -424,6 +427,95 @@ __global__ __launch_bounds__(256) void qp_kernel(MatParams mp0, const double *__
 
 // ------------------------------------------------------------------ phase 2
 // ------------------------------------------------------------------ phase 2
+// P[3 m + i] = sum_j (dxi_m/dx_j) (detJ sigma)_ij of one point from dxi/dx (9) and detJ
+// sigma (s00 s11 s22 s01 s02 s12)
+__device__ __forceinline__ void traction_point_tensor(const double *ix, const double *S, double (&P)[9]) {
+    const double Si[3][3] = {{S[0], S[3], S[4]}, {S[3], S[1], S[5]}, {S[4], S[5], S[2]}};
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) P[3 * m + i] = ix[m] * Si[i][0] + ix[3 + m] * Si[i][1] + ix[6 + m] * Si[i][2];
+}
+
+// Points and element tractions of dense elements, a workgroup to the EPB = 64 / G elements
+// whose points fill its first wave (G <= 64).  The nodes' X and x are staged in LDS once an
+// element; the points' tensors go to LDS and the tractions are contracted from there, as
+// traction_kernel does (same sums in the same order), so the records leave out detJ sigma and
+// detJ, and a residual pass has none.  Bound by the latency of its serial sums.  Time, points
+// and tractions apart -> here (us; elements): 10 nodes, 8 points (3,072) 28 -> 16, (24,576) 77 ->
+// 36; 20 nodes, 14 points (3,072) 35 -> 23; 35 nodes, 31 points (4,374) 87 -> 56.
+// LDS: X and x [EPB npe][6] | P [EPB G][9].
+template <bool TANGENT, bool GEN>
+__global__ __launch_bounds__(256) void qp_traction_kernel(MatParams mp0, const double *__restrict__ points,
+                                                         const int32_t *__restrict__ elements,
+                                                         const double *__restrict__ Eulerx,
+                                                         const double *__restrict__ Jm,
+                                                         const double *__restrict__ JmT, int NP,
+                                                         const double *__restrict__ w, int G, int64_t nelem, int npe,
+                                                         int update, double *__restrict__ qp,
+                                                         int32_t *__restrict__ status,
+                                                         const int32_t *__restrict__ elem_mat,
+                                                         const double *__restrict__ mat_table,
+                                                         double *__restrict__ te) {
+    extern __shared__ double qsm[];
+    const int EPB = 64 / G;
+    const int64_t e0 = (int64_t)blockIdx.x * EPB;
+    const int ne = (int)min((int64_t)EPB, nelem - e0);
+    if (ne <= 0) return;
+    double *sX = qsm, *sP = qsm + EPB * npe * 6;
+    const int tid = threadIdx.x, NT = blockDim.x;
+    const int32_t *conn = elements + e0 * npe;
+    for (int t = tid; t < ne * npe * 3; t += NT) {
+        const int n = t / 3, c = t - 3 * n;
+        const int64_t nd = conn[n];
+        sX[6 * n + c] = points[3 * nd + c];
+        sX[6 * n + 3 + c] = Eulerx[3 * nd + c];
+    }
+    __syncthreads();
+    if (tid < 64) {   // the points' wave
+        const int el = tid / G;
+        const bool valid = el < ne;
+        const int64_t e = valid ? e0 + el : e0;
+        const int g = valid ? tid - el * G : 0;
+        const MatParams mp = element_material(mp0, e, elem_mat, mat_table);
+        double PX[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, Px[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+        const double *xe = sX + (valid ? el : 0) * npe * 6;
+#pragma unroll 5
+        for (int a = 0; a < npe; ++a) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const double jm = Jm[((int64_t)i * npe + a) * G + g];
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    PX[3 * i + c] += jm * xe[6 * a + c];
+                    Px[3 * i + c] += jm * xe[6 * a + 3 + c];
+                }
+            }
+        }
+        double pv[15];
+        qp_point<TANGENT, GEN>(mp, PX, Px, w[g], update, valid,
+                               qp ? qp + e * (int64_t)G * (TANGENT ? QS : QS_RES) + g : nullptr, G, status, false, true, pv);
+        if (valid) {
+            double P[9];
+            traction_point_tensor(pv, pv + 9, P);
+#pragma unroll
+            for (int mi = 0; mi < 9; ++mi) sP[tid * 9 + mi] = P[mi];
+        }
+    }
+    __syncthreads();
+    for (int t = tid; t < ne * 3 * npe; t += NT) {
+        const int te_el = t / (3 * npe), idx = t - te_el * 3 * npe, a = idx / 3, i = idx - 3 * a;
+        const double *P = sP + te_el * G * 9 + i;
+        double acc = 0.0;
+#pragma unroll 4
+        for (int q = 0; q < G; ++q) {
+            const double *jt = JmT + (int64_t)q * 3 * NP + a;
+            acc += jt[0] * P[q * 9] + jt[NP] * P[q * 9 + 3] + jt[2 * NP] * P[q * 9 + 6];
+        }
+        te[e0 * 3 * npe + t] = acc;
+    }
+}
+
 }  // namespace fl
 #include "fl_stiffness.hpp"
 #include "fl_stiffness_bf16.hpp"
@@ -1048,6 +1140,52 @@ static int launch_qp_sf(const MatParams &mp, const double *points, const int32_t
     return FL_E_ARG;
 }
 
+// Points of a dense element: with their tractions where a wave holds an element's points and
+// LDS its nodes (64 KB), else the points alone (traction_kernel follows)
+static size_t points_lds(int G, int npe) { return sizeof(double) * (64 / G) * ((size_t)npe * 6 + (size_t)G * 9); }
+static bool points_fused(int G, int npe) { return G <= 64 && points_lds(G, npe) <= 64 * 1024; }
+
+template <bool TANGENT, bool GEN>
+static int launch_points_t(const MatParams &mp, const double *points, const int32_t *elements, const double *Eulerx,
+                           const double *Jm, const double *JmT, int NP, const double *w, int G, int64_t nelem, int npe,
+                           int update, double *qp, int32_t *status, const int32_t *elem_mat, const double *mat_table,
+                           double *te, hipStream_t st) {
+    if (points_fused(G, npe)) {
+        const int64_t groups = (nelem + 64 / G - 1) / (64 / G);
+        // three more waves share the tractions' sums where all workgroups are on the chip at
+        // once (four a CU: 375 groups of 35 nodes 23 us against 29 with one wave); beyond that
+        // they only take the place of other workgroups (2,187 groups 63 against 56)
+        qp_traction_kernel<TANGENT, GEN><<<(unsigned)groups, groups <= 1024 ? 256 : 64, points_lds(G, npe), st>>>(
+            mp, points, elements, Eulerx, Jm, JmT, NP, w, G, nelem, npe, update, TANGENT ? qp : nullptr, status,
+            elem_mat, mat_table, te);
+    } else {
+        const int64_t nq = nelem * G;
+        qp_kernel<TANGENT, GEN><<<(unsigned)((nq + 255) / 256), 256, 0, st>>>(
+            mp, points, elements, Eulerx, Jm, w, G, nelem, npe, update, qp, status, elem_mat, mat_table);
+    }
+    FL_LAUNCH_CHECK();
+    return 0;
+}
+
+template <bool TANGENT, typename... A>
+static int launch_points(const MatParams &mp, A... a) {
+    return general_law(mp.material) ? launch_points_t<TANGENT, true>(mp, a...)
+                                    : launch_points_t<TANGENT, false>(mp, a...);
+}
+
+template <bool TANGENT>
+static int launch_traction(const double *JmT, int NP, const double *qp, int npe, int G, int64_t nelem, double *te,
+                           hipStream_t st) {
+    const size_t lds = (size_t)G * 9 * 8;
+    if (lds > 64 * 1024)
+        FL_HIP_CHECK(hipFuncSetAttribute((const void *)traction_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         (int)lds));
+    traction_kernel<<<(unsigned)nelem, 256, lds, st>>>(JmT, NP, qp, TANGENT ? QS : QS_RES, TANGENT ? Q_S : QR_S, npe, G,
+                                                       te);
+    FL_LAUNCH_CHECK();
+    return 0;
+}
+
 // the FP32 tangent takes the factorised kernel unless a form other than the default
 // factorised one is selected (FL_TUNE_STIFF_SF 3 and 5 are FP64-only forms: dense there)
 static bool sf32_form() {
@@ -1468,9 +1606,9 @@ static int df_assemble(int32_t material, const double *params, const int32_t *el
     const int NP = padded_np(npe);
     const MatParams mp = mat_params(material, params);
     prof_begin(st, PROF_DF_ASSEMBLE);
-    // status cleared by a kernel, not a memset node, so the call can be graph-captured
-    clear_status_kernel<<<1, 64, 0, st>>>(status);
-    transpose_jm_kernel<<<(G * 3 * NP + 255) / 256, 256, 0, st>>>(Jm, npe, G, NP, w.JmT);
+    // the factorised contractions do not read Jm^T
+    const int gj = use_sf || use_sf32 ? 0 : G;
+    prepare_kernel<<<max(1, (gj * 3 * NP + 255) / 256), 256, 0, st>>>(Jm, npe, gj, NP, w.JmT, status);
     FL_LAUNCH_CHECK();
     const int64_t nq = nelem * G;
     // element-interior rows straight from the default factorised kernel into V (and their
@@ -1487,13 +1625,9 @@ static int df_assemble(int32_t material, const double *params, const int32_t *el
                                           node_elem_ptr, fuse_interior ? T : nullptr);
         if (rq) return rq;
     } else {
-        if (general_law(material))
-            qp_kernel<true, true><<<(unsigned)((nq + 255) / 256), 256, 0, st>>>(
-                mp, points, elements, Eulerx, Jm, AllGauss, G, nelem, npe, update, w.qp, status, elem_mat, mat_table);
-        else
-            qp_kernel<true, false><<<(unsigned)((nq + 255) / 256), 256, 0, st>>>(
-                mp, points, elements, Eulerx, Jm, AllGauss, G, nelem, npe, update, w.qp, status, elem_mat, mat_table);
-        FL_LAUNCH_CHECK();
+        const int rq = launch_points<true>(mp, points, elements, Eulerx, Jm, w.JmT, NP, AllGauss, G, nelem, npe,
+                                           update, w.qp, status, elem_mat, mat_table, w.te, st);
+        if (rq) return rq;
     }
     prof_mark(st);
     // the factorised blocks are stored in tensor node order: tensor_of_l of the basis table,
@@ -1527,13 +1661,9 @@ static int df_assemble(int32_t material, const double *params, const int32_t *el
                        : launch_stiffness_bf16(NP, w.JmT, w.qp, npe, G, nelem, (float *)w.Ke, st);
     if (rc) return rc;
     prof_mark(st);
-    if (!sf_ok) {
-        const size_t lds_tr = (size_t)G * 9 * 8;
-        if (lds_tr > 64 * 1024)
-            FL_HIP_CHECK(hipFuncSetAttribute((const void *)traction_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             (int)lds_tr));
-        traction_kernel<<<(unsigned)nelem, 256, lds_tr, st>>>(w.JmT, NP, w.qp, QS, Q_S, npe, G, w.te);
-        FL_LAUNCH_CHECK();
+    if (!sf_ok && !points_fused(G, npe)) {
+        const int rt = launch_traction<true>(w.JmT, NP, w.qp, npe, G, nelem, w.te, st);
+        if (rt) return rt;
     }
     if (update != 1) {
         const int64_t nte = nelem * 3 * npe;
@@ -1654,32 +1784,23 @@ static int df_residual(int32_t material, const double *params, const int32_t *el
     const int NP = padded_np(npe);
     const MatParams mp = mat_params(material, params);
     if (profile) prof_begin(st, PROF_DF_RESIDUAL);
-    clear_status_kernel<<<1, 64, 0, st>>>(status);
+    const int gj = sf_ok ? 0 : G;
+    prepare_kernel<<<max(1, (gj * 3 * NP + 255) / 256), 256, 0, st>>>(Jm, npe, gj, NP, w.JmT, status);
+    FL_LAUNCH_CHECK();
     if (sf_ok) {
         // no records: the tractions are contracted in the point kernel
         const int rq = launch_qp_sf<false>(mp, points, elements, Eulerx, tensor_basis, AllGauss, npe, G, nelem, 1,
                                            nullptr, status, elem_mat, mat_table, st, 0, w.te);
         if (rq) return rq;
     } else {
-        transpose_jm_kernel<<<(G * 3 * NP + 255) / 256, 256, 0, st>>>(Jm, npe, G, NP, w.JmT);
-        FL_LAUNCH_CHECK();
-        const int64_t nq = nelem * G;
-        if (general_law(material))
-            qp_kernel<false, true><<<(unsigned)((nq + 255) / 256), 256, 0, st>>>(
-                mp, points, elements, Eulerx, Jm, AllGauss, G, nelem, npe, 1, w.qp, status, elem_mat, mat_table);
-        else
-            qp_kernel<false, false><<<(unsigned)((nq + 255) / 256), 256, 0, st>>>(
-                mp, points, elements, Eulerx, Jm, AllGauss, G, nelem, npe, 1, w.qp, status, elem_mat, mat_table);
-        FL_LAUNCH_CHECK();
+        const int rq = launch_points<false>(mp, points, elements, Eulerx, Jm, w.JmT, NP, AllGauss, G, nelem, npe, 1,
+                                            w.qp, status, elem_mat, mat_table, w.te, st);
+        if (rq) return rq;
     }
     if (profile) prof_mark(st);
-    if (!sf_ok) {
-        const size_t lds_tr = (size_t)G * 9 * 8;
-        if (lds_tr > 64 * 1024)
-            FL_HIP_CHECK(hipFuncSetAttribute((const void *)traction_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             (int)lds_tr));
-        traction_kernel<<<(unsigned)nelem, 256, lds_tr, st>>>(w.JmT, NP, w.qp, QS_RES, QR_S, npe, G, w.te);
-        FL_LAUNCH_CHECK();
+    if (!sf_ok && !points_fused(G, npe)) {
+        const int rt = launch_traction<false>(w.JmT, NP, w.qp, npe, G, nelem, w.te, st);
+        if (rt) return rt;
     }
     if (profile) prof_mark(st);
     gather_traction_kernel<<<(unsigned)((3 * nnode + 255) / 256), 256, 0, st>>>(npe, node_elem_ptr, node_elem, w.te,

@@ -46,16 +46,6 @@ struct SfLayout {
     static constexpr int INTS = 4 + Q3 + 2 * N3 + (Q3 % 2);   // 8-byte aligned
 };
 
-// P[3 m + i] = sum_j (dxi_m/dx_j) (detJ sigma)_ij of one point from dxi/dx (9) and detJ
-// sigma (s00 s11 s22 s01 s02 s12)
-__device__ __forceinline__ void traction_point_tensor(const double *ix, const double *S, double (&P)[9]) {
-    const double Si[3][3] = {{S[0], S[3], S[4]}, {S[3], S[1], S[5]}, {S[4], S[5], S[2]}};
-#pragma unroll
-    for (int m = 0; m < 3; ++m)
-#pragma unroll
-        for (int i = 0; i < 3; ++i) P[3 * m + i] = ix[m] * Si[i][0] + ix[3 + m] * Si[i][1] + ix[6 + m] * Si[i][2];
-}
-
 // The sum factorisation of a point kernel, shared by qp_sf_kernel (X and x, NF = 6) and
 // mf_element_kernel (a dof vector, NF = 3): a workgroup of 128 threads (256 for 6^3 points)
 // for the EPB elements whose points fill it, a point per thread.  Gradients of the NF

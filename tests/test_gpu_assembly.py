@@ -201,6 +201,52 @@ def test_element_form_rules(cuda, et, p, norder):
         lib.fl_set_tuning(_lib.FL_TUNE_STIFF_SF, 0)
 
 
+@pytest.mark.parametrize("p,n", [(1, 1), (1, 3), (2, 1), (3, 2), (4, 1)])
+def test_dense_points_and_tractions(cuda, p, n):
+    """Points and tractions of dense elements in one kernel: 64 to 2 elements a workgroup, with
+    and without a rest.  T against the oracle; the assembly's T is the residual pass's."""
+    import torch
+    from florence_amd.assembly import DeviceMeshData, assemble_device, residual_device
+    m = cube_mesh("tet", p, n, jitter=0.05, seed=80 + p)
+    fs = function_space(m, p)
+    mat = MooneyRivlin(3, mu1=0.5, mu2=0.5, lamb=20.0)
+    x = deformed(m.points, 0.04 / n, seed=81 + p)
+    dm = DeviceMeshData(m, fs)
+    R, st = residual_device(dm, mat, x)
+    R = R.clone()
+    assert int(st[0].item()) == 0
+    _, T, _ = assemble_device(dm, mat, x)
+    torch.cuda.synchronize()
+    Tr = O.residual_only(m.points, m.elements, x, fs.Jm, fs.AllGauss, mat)
+    assert np.abs(R.cpu().numpy() - Tr).max() <= RTOL * np.abs(Tr).max()
+    assert np.array_equal(R.cpu().numpy(), T.cpu().numpy())
+
+
+@pytest.mark.parametrize("p,copies", [(1, 420), (2, 60), (4, 14)])
+def test_dense_points_many_groups(cuda, p, copies):
+    """Above 1,024 workgroups the points' kernel runs without its helping waves: disconnected
+    copies of a mesh of 162 tets give, copy by copy, the T of the one, bit for bit."""
+    import torch
+    from florence_amd.assembly import DeviceMeshData, residual_device
+    m = cube_mesh("tet", p, 3, jitter=0.05, seed=90 + p)
+    fs = function_space(m, p)
+    mat = MooneyRivlin(3, mu1=0.5, mu2=0.5, lamb=20.0)
+    x = deformed(m.points, 0.02, seed=91 + p)
+    one, st = residual_device(DeviceMeshData(m, fs), mat, x)
+    one = one.clone()
+    assert int(st[0].item()) == 0
+    big = cube_mesh("tet", p, 3, jitter=0.05, seed=90 + p)
+    groups = -(-copies * m.nelem // (64 // fs.AllGauss.shape[0]))
+    assert groups > 1024
+    big.points = np.ascontiguousarray(np.tile(m.points, (copies, 1)))
+    big.elements = np.concatenate([np.asarray(m.elements) + m.nnode * c for c in range(copies)])
+    big.nelem, big.nnode = copies * m.nelem, copies * m.nnode
+    T, st = residual_device(DeviceMeshData(big, fs), mat, np.tile(x, (copies, 1)))
+    torch.cuda.synchronize()
+    assert int(st[0].item()) == 0
+    assert torch.equal(T.reshape(copies, -1), one.reshape(1, -1).expand(copies, -1))
+
+
 @pytest.mark.parametrize("p", [1, 2, 3, 4])
 def test_sum_factorised_equals_dense(cuda, p):
     """Tensor-product hexes: the sum-factorised point, block and traction kernels (default
