@@ -818,11 +818,13 @@ __global__ void gather_traction_kernel(int npe, const int32_t *__restrict__ node
 // element).  Class 0 (the smallest neighbour count) whose degree equals npe holds
 // element-interior nodes only (a node of two distinct elements has more than npe
 // neighbours): gather_single_kernel.  Elements of at most 64 nodes: one wave per node
-// in every class, <64, 8, 2> for npe <= 14 and <64, 4, 9> up to 64.  Larger elements:
+// in every class, <64, 8, 2> for npe <= 14, <64, 8, 3> up to 21, <64, 4, 5> up to 35 and <64, 4,
+// 9> up to 64: no more loads a lane than an element has (in <64, 4, 9>, us: 20 nodes, 3,072
+// elements 72 -> 62, 35 nodes, 48 elements 61 -> 59, 4,374 246 -> 241).  Larger elements:
 // the other classes use <256, EB, 5> with EB = 2, 4 or 8 as the class's degree suggests
 // its nodes' element count (deg <= 2 npe, <= 4 npe, more: chunks longer than that only
 // cost registers), class 0 one wave per node, <64, 2, 18>.
-enum GatherForm { G_SINGLE, G_W8X2, G_W4X9, G_W2X18, G_WIDE1, G_WIDE2, G_WIDE4, G_WIDE8 };
+enum GatherForm { G_SINGLE, G_W8X2, G_W8X3, G_W4X5, G_W4X9, G_W2X18, G_WIDE1, G_WIDE2, G_WIDE4, G_WIDE8 };
 
 // FL_TUNE_GATHER: bit 0 = the wide classes one element at a time (<256, 1, 5>), bit 1 =
 // the single-element class through gather_kernel<64, 2, 18>
@@ -831,6 +833,8 @@ static GatherForm gather_form(int b, int deg, int npe) {
     if (b == 0 && deg == npe && !(t & 2)) return G_SINGLE;
     // up to 64 nodes an element's 9 npe values fill at most 9 loads of one wave
     if (npe <= 14) return G_W8X2;
+    if (npe <= 21) return G_W8X3;
+    if (npe <= 35) return G_W4X5;
     if (npe <= 64) return G_W4X9;
     if (b > 0) {
         if (t & 1) return G_WIDE1;
@@ -841,8 +845,8 @@ static GatherForm gather_form(int b, int deg, int npe) {
 
 static int gather_eb(GatherForm f) {
     switch (f) {
-        case G_W8X2: case G_WIDE8: return 8;
-        case G_W4X9: case G_WIDE4: return 4;
+        case G_W8X2: case G_W8X3: case G_WIDE8: return 8;
+        case G_W4X5: case G_W4X9: case G_WIDE4: return 4;
         case G_W2X18: case G_WIDE2: return 2;
         default: return 1;
     }
@@ -853,6 +857,25 @@ static int gather_eb(GatherForm f) {
 static size_t gather_lds_bytes(GatherForm f, int deg, int npe) {
     if (f == G_SINGLE) return (size_t)8 * npe + (size_t)72 * npe + 16;
     return (size_t)(gather_eb(f) * npe + deg + 1) / 2 * 8 + (size_t)deg * 9 * 8 + 16;
+}
+
+// One past the last class that shares class b's launch, with the greatest degree in *deg:
+// for elements of at most 64 nodes (a wave a node), the classes whose LDS leaves a CU all its
+// 32 waves, or whose nodes are all on the chip at once.  A class of less LDS has no use for a
+// launch of its own then (the gather of 3,072 elements of 10 nodes 28 -> 23 us, 162 of 20 36 ->
+// 21, 48 of 35 59 -> 30, 750 of 35 80 -> 63; in one launch at any size the least class would
+// run at the greatest's occupancy).
+static int gather_classes(const int32_t *bucket_offsets, const int32_t *bucket_degree, int b, int npe, int *deg) {
+    int next = b + 1;
+    if (npe > 64 || tuning_value(TUNE_GATHER, 0) != 0) return next;
+    for (; next < FL_GATHER_BUCKETS; ++next) {
+        if (bucket_offsets[next + 1] == bucket_offsets[next]) continue;
+        const int d = *deg > bucket_degree[next] ? *deg : bucket_degree[next];
+        const size_t lds = gather_lds_bytes(gather_form(1, d, npe), d, npe), cu = 160 * 1024 / (lds ? lds : 1);
+        if (cu < 32 && bucket_offsets[next + 1] - bucket_offsets[b] > (int64_t)(256 * cu)) break;
+        *deg = d;
+    }
+    return next;
 }
 
 static int padded_np(int npe) {
@@ -1252,6 +1275,12 @@ static int launch_gather(int b, int32_t nb, const int32_t *elements, int npe, co
             return 0;
         case G_W8X2:
             return launch_gather_t<KT, 64, 8, 2, VT>(nb, lds, elements, npe, order, node_elem_ptr, node_elem, nbr_ptr,
+                                                     nbrs, indptr, Ke, te, deg, ranks, kperm, kinv, eslot, V, T, status, st);
+        case G_W8X3:
+            return launch_gather_t<KT, 64, 8, 3, VT>(nb, lds, elements, npe, order, node_elem_ptr, node_elem, nbr_ptr,
+                                                     nbrs, indptr, Ke, te, deg, ranks, kperm, kinv, eslot, V, T, status, st);
+        case G_W4X5:
+            return launch_gather_t<KT, 64, 4, 5, VT>(nb, lds, elements, npe, order, node_elem_ptr, node_elem, nbr_ptr,
                                                      nbrs, indptr, Ke, te, deg, ranks, kperm, kinv, eslot, V, T, status, st);
         case G_W4X9:
             return launch_gather_t<KT, 64, 4, 9, VT>(nb, lds, elements, npe, order, node_elem_ptr, node_elem, nbr_ptr,
@@ -1679,22 +1708,25 @@ static int df_assemble(int32_t material, const double *params, const int32_t *el
         prof_mark(st);
         return 0;
     }
-    for (int b = fuse_interior ? 1 : 0; b < FL_GATHER_BUCKETS; ++b) {
-        const int32_t nb = bucket_offsets[b + 1] - bucket_offsets[b];
+    for (int b = fuse_interior ? 1 : 0, next; b < FL_GATHER_BUCKETS; b = next) {
+        int dg = bucket_degree[b];
+        next = gather_classes(bucket_offsets, bucket_degree, b, npe, &dg);
+        const int32_t nb = bucket_offsets[next] - bucket_offsets[b];
         if (nb <= 0) continue;
+        // several classes: the form of one of more than one element
+        const int fb = next > b + 1 ? 1 : b;
         int rc2 = 0;
         const int32_t *ord = node_order + bucket_offsets[b];
-        const int dg = bucket_degree[b];
         if (precision == FL_PREC_FP64)
-            rc2 = launch_gather<double, double>(b, nb, elements, npe, ord, node_elem_ptr, node_elem, node_nbr_ptr,
+            rc2 = launch_gather<double, double>(fb, nb, elements, npe, ord, node_elem_ptr, node_elem, node_nbr_ptr,
                                                 node_nbrs, indptr, (const double *)w.Ke, w.te, dg, ranks, kperm,
                                                 kinv, eslot, V, T, status, st);
         else if (!v32)
-            rc2 = launch_gather<float, double>(b, nb, elements, npe, ord, node_elem_ptr, node_elem, node_nbr_ptr,
+            rc2 = launch_gather<float, double>(fb, nb, elements, npe, ord, node_elem_ptr, node_elem, node_nbr_ptr,
                                                node_nbrs, indptr, (const float *)w.Ke, w.te, dg, ranks, kperm,
                                                kinv, eslot, V, T, status, st);
         else
-            rc2 = launch_gather<float, float>(b, nb, elements, npe, ord, node_elem_ptr, node_elem, node_nbr_ptr,
+            rc2 = launch_gather<float, float>(fb, nb, elements, npe, ord, node_elem_ptr, node_elem, node_nbr_ptr,
                                               node_nbrs, indptr, (const float *)w.Ke, w.te, dg, ranks, kperm,
                                               kinv, eslot, reinterpret_cast<float *>(V), T, status, st);
         if (rc2) return rc2;

@@ -247,6 +247,28 @@ def test_dense_points_many_groups(cuda, p, copies):
     assert torch.equal(T.reshape(copies, -1), one.reshape(1, -1).expand(copies, -1))
 
 
+@pytest.mark.parametrize("p,copies", [(1, 1000), (2, 40), (3, 12), (4, 10)])
+def test_gather_launches(cuda, p, copies):
+    """A small mesh's degree classes are gathered in one launch, a large one's apart:
+    disconnected copies of a mesh of 162 tets give, copy by copy, the values of the one."""
+    import torch
+    from florence_amd.assembly import DeviceMeshData, assemble_device
+    m = cube_mesh("tet", p, 3, jitter=0.05, seed=90 + p)
+    fs = function_space(m, p)
+    mat = MooneyRivlin(3, mu1=0.5, mu2=0.5, lamb=20.0)
+    x = deformed(m.points, 0.02, seed=91 + p)
+    V, T, _ = (t.cpu().numpy() for t in assemble_device(DeviceMeshData(m, fs), mat, x))
+    big = cube_mesh("tet", p, 3, jitter=0.05, seed=90 + p)
+    big.points = np.ascontiguousarray(np.tile(m.points, (copies, 1)))
+    big.elements = np.concatenate([np.asarray(m.elements) + m.nnode * c for c in range(copies)])
+    big.nelem, big.nnode = copies * m.nelem, copies * m.nnode
+    Vb, Tb, st = assemble_device(DeviceMeshData(big, fs), mat, np.tile(x, (copies, 1)))
+    torch.cuda.synchronize()
+    assert int(st[0].item()) == 0
+    assert np.array_equal(Vb.cpu().numpy().reshape(copies, -1), np.broadcast_to(V, (copies, V.size)))
+    assert np.array_equal(Tb.cpu().numpy().reshape(copies, -1), np.broadcast_to(T, (copies, T.size)))
+
+
 @pytest.mark.parametrize("p", [1, 2, 3, 4])
 def test_sum_factorised_equals_dense(cuda, p):
     """Tensor-product hexes: the sum-factorised point, block and traction kernels (default
