@@ -78,6 +78,31 @@ __device__ inline void node_spmv(const int32_t *__restrict__ indptr, const int32
         if (!free_mask[3 * a + i]) q[i] = 0.0;
 }
 
+// A thread per dof: a wave takes 21 nodes, lanes 3 n + i, i < 3, node n's component i (lane 63
+// none), so that vector accesses are contiguous and a level of 10^5 nodes fills the chip.
+constexpr int DOF_NB = SV_T / 64 * 21;   // nodes of a workgroup
+static unsigned nb_dof(int64_t nnode) { return (unsigned)((nnode + DOF_NB - 1) / DOF_NB); }
+struct DofLane {
+    int64_t a;    // node, in range also where !on
+    int n, i;     // node within the wave, component
+    bool on;
+};
+__device__ inline DofLane dof_lane(int64_t nnode) {
+    DofLane l;
+    const int lane = threadIdx.x & 63;
+    l.n = lane / 3;
+    l.i = lane - 3 * l.n;
+    const int64_t a = ((int64_t)blockIdx.x * (SV_T / 64) + (threadIdx.x >> 6)) * 21 + l.n;
+    l.on = lane < 63 && a < nnode;
+    l.a = a < nnode ? a : nnode - 1;
+    return l;
+}
+// component i of P r at the lane's node, p: row i of P, r: the lane's component (bj_apply's sum)
+__device__ inline double dof_apply(const double (&p)[3], double r, const DofLane &l) {
+    const double r0 = __shfl(r, 3 * l.n, 64), r1 = __shfl(r, 3 * l.n + 1, 64), r2 = __shfl(r, 3 * l.n + 2, 64);
+    return p[0] * r0 + p[1] * r1 + p[2] * r2;
+}
+
 // Chebyshev start: r = b (if b given), d = D^-1 r / theta, x = d (fresh) or x += d.
 __global__ __launch_bounds__(SV_T) void cheb_init_kernel(int64_t nnode, const double *__restrict__ P,
                                                          const double *__restrict__ b, double *__restrict__ r,
@@ -103,6 +128,8 @@ __global__ __launch_bounds__(SV_T) void cheb_init_kernel(int64_t nnode, const do
 // One Chebyshev step: r -= A d_old; d_new = c1 d_old + c2 D^-1 r; x += d_new.
 // c2 = 0 and x = d_new = nullptr: only the residual update r -= A d.  LPN lanes per node
 // (64 on the fine level; 32 on the coarse levels, whose nodes have fewer neighbours).
+// 15,625 p = 2 hex nodes, FP32 values: 11.9 us with the update by one lane after the row's
+// sum, 10.1 with its operands loaded before it by three.
 template <typename VT, int LPN>
 __global__ __launch_bounds__(64 * SP_W) void cheb_step_kernel(const int32_t *__restrict__ indptr,
                                                               const int32_t *__restrict__ nbr_ptr,
@@ -116,30 +143,36 @@ __global__ __launch_bounds__(64 * SP_W) void cheb_step_kernel(const int32_t *__r
     const int grp = threadIdx.x / LPN, lane = threadIdx.x % LPN;
     const int64_t a = (int64_t)blockIdx.x * (64 * SP_W / LPN) + grp;
     if (a >= nnode) return;
+    // the group's first three lanes take a component each; what they need besides the row is
+    // in flight over the row's sum
+    const int i = lane < 3 ? lane : 2;
+    const int64_t g = 3 * a + i;
+    const double r0 = r[g], dv = d_old[g];
+    double xv = 0.0, p[3] = {0.0, 0.0, 0.0};
+    if (d_new) {
+        xv = x[g];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) p[k] = P[3 * g + k];
+    }
     double q[3];
     node_spmv<VT, LPN>(indptr, nbr_ptr, nbrs, V, free_mask, d_old, a, lane, q);
-    if (lane != 0) return;
-    double rv[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        rv[i] = r[3 * a + i] - q[i];
-        r[3 * a + i] = rv[i];
-    }
+    const double rv = r0 - (i == 0 ? q[0] : (i == 1 ? q[1] : q[2]));
+    const int base = (threadIdx.x & 63) - lane;
+    const double v0 = __shfl(rv, base, 64), v1 = __shfl(rv, base + 1, 64), v2 = __shfl(rv, base + 2, 64);
+    if (lane >= 3) return;
+    r[g] = rv;
     if (!d_new) return;
-    double z[3];
-    bj_apply(P, a, rv, z);
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        const double dn = c1 * d_old[3 * a + i] + c2 * z[i];
-        d_new[3 * a + i] = dn;
-        x[3 * a + i] += dn;
-    }
+    const double dn = c1 * dv + c2 * (p[0] * v0 + p[1] * v1 + p[2] * v2);
+    d_new[g] = dn;
+    x[g] = xv + dn;
 }
 
 // The matrix-free product's node sums: q = sum of the element vectors ye of node a's
 // elements (node_elem: element * npe + local, ascending element order), 0 on fixed dofs.
 // With q_out: q_out = q.  Otherwise as cheb_step_kernel: r -= q and, with d_new, the
-// Chebyshev update.
+// Chebyshev update.  Bound by load latency and the 31 MB of vectors, blocks and element
+// values: 117,649 nodes of p = 4 hexes, a thread a node and one element at a time 9.9 us, a
+// thread a dof with four elements and the update's operands in flight 8.7.
 __global__ __launch_bounds__(SV_T) void mf_node_kernel(int64_t nnode, const int32_t *__restrict__ node_elem_ptr,
                                                        const int32_t *__restrict__ node_elem,
                                                        const double *__restrict__ ye,
@@ -148,38 +181,40 @@ __global__ __launch_bounds__(SV_T) void mf_node_kernel(int64_t nnode, const int3
                                                        double *__restrict__ d_new, double *__restrict__ r,
                                                        double *__restrict__ x, double *__restrict__ q_out, double c1,
                                                        double c2) {
-    const int64_t a = (int64_t)blockIdx.x * SV_T + threadIdx.x;
-    if (a >= nnode) return;
-    double q[3] = {0.0, 0.0, 0.0};
-    for (int32_t j = node_elem_ptr[a]; j < node_elem_ptr[a + 1]; ++j) {
-        const double *v = ye + 3 * (int64_t)node_elem[j];
-        q[0] += v[0];
-        q[1] += v[1];
-        q[2] += v[2];
+    const DofLane l = dof_lane(nnode);
+    const int64_t g = 3 * l.a + l.i;
+    const int32_t j1 = node_elem_ptr[l.a + 1];
+    // what the update needs besides the sum is in flight over it
+    const bool fr = free_mask[g] != 0;
+    double r0 = 0.0, dv = 0.0, xv = 0.0, p[3] = {0.0, 0.0, 0.0};
+    if (!q_out) r0 = r[g];
+    if (!q_out && d_new) {
+        dv = d_old[g];
+        xv = x[g];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) p[k] = P[3 * g + k];
     }
+    double q = 0.0;
+    for (int32_t j = node_elem_ptr[l.a]; j < j1; j += 4) {   // four elements' values at a time
+        double v[4];
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
-        if (!free_mask[3 * a + i]) q[i] = 0.0;
+        for (int u = 0; u < 4; ++u) v[u] = j + u < j1 ? ye[3 * (int64_t)node_elem[j + u] + l.i] : 0.0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (j + u < j1) q += v[u];
+    }
+    if (!fr) q = 0.0;
     if (q_out) {
-#pragma unroll
-        for (int i = 0; i < 3; ++i) q_out[3 * a + i] = q[i];
+        if (l.on) q_out[g] = q;
         return;
     }
-    double rv[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        rv[i] = r[3 * a + i] - q[i];
-        r[3 * a + i] = rv[i];
-    }
+    const double rv = r0 - q, z = dof_apply(p, rv, l);
+    if (!l.on) return;
+    r[g] = rv;
     if (!d_new) return;
-    double z[3];
-    bj_apply(P, a, rv, z);
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        const double dn = c1 * d_old[3 * a + i] + c2 * z[i];
-        d_new[3 * a + i] = dn;
-        x[3 * a + i] += dn;
-    }
+    const double dn = c1 * dv + c2 * z;
+    d_new[g] = dn;
+    x[g] = xv + dn;
 }
 
 // Sum of part[stride * i + col], i < n, by one wave: lane l takes i = l, l + 64, ... in
@@ -343,7 +378,9 @@ __global__ __launch_bounds__(64 * SP_W) void restrict_kernel(int64_t nnode_c, co
     }
 }
 
-// d[f] = sum_j P_w[j] e_coarse[P_idx[j]] (masked by the fine free dofs); x += d
+// d[f] = sum_j P_w[j] e_coarse[P_idx[j]] (masked by the fine free dofs); x += d.  Bound by the
+// latency of its chain of loads: 117,649 nodes one coarse node at a time 15.1 us, four 12.0 (a
+// thread a dof reads every weight three times: 16.7).
 __global__ __launch_bounds__(SV_T) void prolong_kernel(int64_t nnode, const int32_t *__restrict__ P_ptr,
                                                        const int32_t *__restrict__ P_idx,
                                                        const double *__restrict__ P_w,
@@ -352,13 +389,25 @@ __global__ __launch_bounds__(SV_T) void prolong_kernel(int64_t nnode, const int3
                                                        double *__restrict__ x) {
     const int64_t f = (int64_t)blockIdx.x * SV_T + threadIdx.x;
     if (f >= nnode) return;
+    const int32_t j1 = P_ptr[f + 1];
     double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-    for (int32_t j = P_ptr[f]; j < P_ptr[f + 1]; ++j) {
-        const int64_t c = P_idx[j];
-        const double w = P_w[j];
-        s0 += w * ec[3 * c];
-        s1 += w * ec[3 * c + 1];
-        s2 += w * ec[3 * c + 2];
+    for (int32_t j = P_ptr[f]; j < j1; j += 4) {   // four coarse nodes' values in flight
+        double w[4], e[4][3];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int32_t jc = j + u < j1 ? j + u : j1 - 1;
+            const int64_t c = P_idx[jc];
+            w[u] = P_w[jc];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) e[u][i] = ec[3 * c + i];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (j + u < j1) {
+                s0 += w[u] * e[u][0];
+                s1 += w[u] * e[u][1];
+                s2 += w[u] * e[u][2];
+            }
     }
     const double v[3] = {free_mask[3 * f] ? s0 : 0.0, free_mask[3 * f + 1] ? s1 : 0.0, free_mask[3 * f + 2] ? s2 : 0.0};
 #pragma unroll
@@ -607,7 +656,7 @@ static int mf_product(const Mg &m, const double *d, double *q_out, const double 
     const FlMgLevel &L = m.lv[0];
     const int rc = mf_element_apply(m.mf, L.free_mask, d, m.st);
     if (rc) return rc;
-    mf_node_kernel<<<nb_v(L.nnode), SV_T, 0, m.st>>>(L.nnode, m.mf.node_elem_ptr, m.mf.node_elem, m.mf.ye,
+    mf_node_kernel<<<nb_dof(L.nnode), SV_T, 0, m.st>>>(L.nnode, m.mf.node_elem_ptr, m.mf.node_elem, m.mf.ye,
                                                      L.free_mask, m.w[0].P, d_old, d_new, m.w[0].r, x, q_out, c1, c2);
     FL_LAUNCH_CHECK();
     return 0;
@@ -906,7 +955,7 @@ int fl_mf_apply(const FlMgMatrixFree *op, const uint8_t *free_mask, const double
     hipStream_t st = as_stream(stream);
     rc = mf_element_apply(mo, free_mask, x, st);
     if (rc) return rc;
-    mf_node_kernel<<<nb_v(mo.nnode), SV_T, 0, st>>>(mo.nnode, mo.node_elem_ptr, mo.node_elem, mo.ye, free_mask,
+    mf_node_kernel<<<nb_dof(mo.nnode), SV_T, 0, st>>>(mo.nnode, mo.node_elem_ptr, mo.node_elem, mo.ye, free_mask,
                                                     nullptr, nullptr, nullptr, nullptr, nullptr, y, 0.0, 0.0);
     FL_LAUNCH_CHECK();
     return 0;
