@@ -56,12 +56,10 @@ def tensor_basis_table(function_space, npe):
         return None
     C = P1 - 2
     f1d = np.zeros((3, 2, P1, Q))
-    for d in range(3):
-        for q in range(Q):
-            pts = z[qi[:, d] == q, d]
-            N, dN = LagrangeGaussLobatto1D(C, float(pts[0]))
-            f1d[d, 0, :, q] = N
-            f1d[d, 1, :, q] = dN
+    # each direction's 1D points, as the first point that holds them has them
+    pts = np.stack([z[np.unique(qi[:, d], return_index=True)[1], d] for d in range(3)])
+    N, dN = LagrangeGaussLobatto1D(C, pts)
+    f1d[:, 0], f1d[:, 1] = N.transpose(1, 0, 2), dN.transpose(1, 0, 2)
     perm = np.asarray(NodeArrangementHex(C))
     if perm.shape != (npe,) or not np.array_equal(np.sort(perm), np.arange(npe)):
         return None

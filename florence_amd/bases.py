@@ -35,18 +35,29 @@ __all__ = [
 
 def LagrangeGaussLobatto1D(C, xi):
     """1D Lagrange bases through the C+2 GLL points and their derivatives at ``xi``
-    (Florence/FunctionSpace/OneDimensional/Line.py:108-132).  Returns (N, dN), each (C+2,)."""
+    (Florence/FunctionSpace/OneDimensional/Line.py:108-132).  Returns (N, dN), each (C+2,),
+    or (C+2,) + xi's shape for an array of points (the same values, point by point)."""
     n = C + 2
     nodes = GaussLobattoQuadrature(n)[0][:, 0]
-    N = np.ones(n)
-    dN = np.zeros(n)
+    xi = np.asarray(xi, dtype=np.float64)
+    N = np.ones((n,) + xi.shape)
+    dN = np.zeros((n,) + xi.shape)
+    diff = [xi - nodes[m] for m in range(n)]
     for a in range(n):
         others = [m for m in range(n) if m != a]
-        denom = np.prod([nodes[a] - nodes[m] for m in others])
-        N[a] = np.prod([xi - nodes[m] for m in others]) / denom
+        denom = 1.0
+        p = np.ones(xi.shape)
+        for m in others:
+            denom = denom * (nodes[a] - nodes[m])
+            p = p * diff[m]
+        N[a] = p / denom
         s = 0.0
         for skip in others:
-            s += np.prod([xi - nodes[m] for m in others if m != skip])
+            p = np.ones(xi.shape)
+            for m in others:
+                if m != skip:
+                    p = p * diff[m]
+            s = s + p
         dN[a] = s / denom
     return N, dN
 

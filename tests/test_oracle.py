@@ -346,3 +346,15 @@ def test_oracle_translation_spread():
     FL = np.swapaxes(np.einsum("egja,eal->egjl", np.einsum("egjk,kag->egja", iX, fs.Jm.astype(L)),
                                x[el].astype(L)), -1, -2)
     assert np.abs(F - FL).max() > 1e-14
+
+
+@pytest.mark.parametrize("p", [1, 2, 3, 4])
+def test_gauss_lobatto_bases_at_many_points(p):
+    """The 1D bases at an array of points are those at each point, bit for bit."""
+    from florence_amd.bases import LagrangeGaussLobatto1D
+    x = np.linspace(-1.0, 1.0, 7).reshape(1, 7) * np.array([[1.0], [0.3]])
+    N, dN = LagrangeGaussLobatto1D(p - 1, x)
+    assert N.shape == dN.shape == (p + 1, 2, 7)
+    for i in np.ndindex(x.shape):
+        n, dn = LagrangeGaussLobatto1D(p - 1, float(x[i]))
+        assert np.array_equal(N[(slice(None),) + i], n) and np.array_equal(dN[(slice(None),) + i], dn)
