@@ -3,7 +3,9 @@
 // Restates the element loop of _GlobalAssemblyDF_ (Florence/FiniteElements/Assembly/
 // _Assembly_/_LowLevelAssemblyDF_.h:69-161) as four device phases:
 //
-//  1. qp_kernel       one thread per (element, quadrature point): gather X, x; the
+//  1. qp_traction_kernel (dense elements of at most 64 points, with phase 3), qp_sf_kernel (tensor-
+//                     product hexes, with phase 3), qp_kernel: one thread per (element,
+//                     quadrature point): gather X, x; the
 //                     kinematics of _KinematicMeasures_.h:64-119 (parent Jacobians,
 //                     adjugate inverses, detJ = w |det dx/dxi|, F); the Neo-Hookean /
 //                     Mooney-Rivlin laws of _NeoHookean_.h:27-51 / _MooneyRivlin_.h:30-70
@@ -11,7 +13,8 @@
 //                     Mooney-Rivlin laws, material_law_gen below).
 //                     Emits per point: dxi/dx (9), the six coupling blocks
 //                     D^{ik}_{jl} = detJ (c_ijkl + delta_ik sigma_jl) (54) and detJ*sigma (6).
-//  2. stiffness_kernel one workgroup per (element, block pair i<=k): the constitutive
+//  2. stiffness_kernel one workgroup per (element, block pair i<=k), stiffness_el_kernel one per
+//                     element, stiffness_rows_kernel and the other factorised forms: the constitutive
 //                     B.H.B^T of _ConstitutiveStiffnessDF_.h:83-134 plus the geometric term
 //                     of _GeometricStiffness_.h:61-100, written per 3x3 displacement block
 //                       K^{ik}_{ab} = sum_{g,j} G_{a,(g,j)} W^{ik}_{b,(g,j)},

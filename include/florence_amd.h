@@ -447,7 +447,8 @@ int fl_profile_enable(int on);
  * 32: v0 2x2/1x1, v1 1x1/2x2, v2 2x1/1x2, v3 1x2/2x1; 48: v0 3x3/1x1, v1 1x3/3x1,
  * v2 3x1/1x3; 64: v0 2x2/2x2, v1 4x4/1x1, v2 4x2/1x2, v3 2x4/2x1, v4 2x1/2x4;
  * 128: v0 default (off-diagonal pairs 4x4/2x2, then the diagonal triangles), v1 one
- * wave per SIMD, all pairs square, v2 off-diagonal pairs 8x2/1x4.  Used by the
+ * wave per SIMD, all pairs square, v2 off-diagonal pairs 8x2/1x4.  In FP64 v0 of up to 16,
+ * 17 to 20 and 33 to 36 nodes is the element form (one workgroup an element).  Used by the
  * autotuner; fl_stiffness_variant_count(c) gives the number of variants of class c
  * (0 for an unknown class).  No reference counterpart. */
 #define FL_TUNE_STIFF_VARIANT_BASE 2
