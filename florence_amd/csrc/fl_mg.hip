@@ -985,6 +985,7 @@ int fl_mg_pcg(const FlMgLevel *levels, int32_t nlevels, int32_t v32, const float
     }
     if (check_every <= 0) check_every = 1;
     Mg m = {};
+    m.st = as_stream(stream);
     m.lv = levels;
     m.nl = nlevels;
     m.v32 = v32 ? 1 : 0;
@@ -1011,7 +1012,6 @@ int fl_mg_pcg(const FlMgLevel *levels, int32_t nlevels, int32_t v32, const float
     m.degree = cheb_degree;
     m.range = cheb_range;
     m.coarse_its = coarse_iterations;
-    m.st = as_stream(stream);
     const int64_t n0 = 3 * levels[0].nnode;
     Carve cv(workspace, workspace_bytes);
     double *rO = cv.take<double>(n0), *rOld = cv.take<double>(n0), *p = cv.take<double>(n0), *q = cv.take<double>(n0);

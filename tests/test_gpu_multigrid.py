@@ -398,3 +398,35 @@ def test_coarse_cg_in_one_launch(cuda):
         lib.fl_set_tuning(_lib.FL_TUNE_CG, 0)
     assert torch.equal(x[1][0], x[2][0])
     assert float(torch.linalg.norm(x[0][0] - x[1][0]) / torch.linalg.norm(x[1][0])) <= 1e-9
+
+
+@pytest.mark.parametrize("records", ["bf16", "fp32"])
+def test_solve_on_a_stream_of_its_own(cuda, records):
+    """Assembly and solve on another stream than the default one, which idles meanwhile: the
+    smoother's rounded copy of the records is made after the assembly that writes them, so
+    the solve is bitwise the default stream's.  (On any other stream the copy would be of
+    the records of the state before.)"""
+    import torch
+    from florence_amd.assembly import DeviceMeshData, assemble_device
+    from florence_amd.multigrid import MultigridSolver
+    m, fs, mat = cube_hex_p4(3)
+    dm = DeviceMeshData(m, fs)
+    x = torch.as_tensor(twisted_state(m, 12.0), device=cuda)
+    x0 = torch.as_tensor(np.ascontiguousarray(m.points), device=cuda)
+    free = torch.as_tensor(np.isnan(clamp_and_twist(m)).ravel().astype(np.uint8), device=cuda)
+    b = torch.as_tensor(np.random.default_rng(2).standard_normal(free.numel()), device=cuda) * free
+
+    def solve():
+        V, _, _ = assemble_device(dm, mat, x)
+        return MultigridSolver(rtol=1e-10, smoother_records=records).Solve(dm, V, free, b, torch.empty_like(b))
+
+    ref = solve()
+    assemble_device(dm, mat, x0)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        torch.cuda._sleep(20000000)   # the assembly starts late
+        got = solve()
+    s.synchronize()
+    assert torch.equal(got, ref)
