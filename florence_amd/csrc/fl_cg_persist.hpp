@@ -29,7 +29,9 @@
 // All workgroups must be resident at once: at most one per CU is launched, one such
 // solve per device runs at a time in a process (persistent_lock), and every wait is bounded: a
 // workgroup that waits longer than wait_ticks raises the abort flag and returns, the others
-// follow, x is left untouched, and the caller solves with the launch-per-step form.
+// follow, and the caller solves with the launch-per-step form.  x is undefined then: where
+// the wait that runs out is one for the last meeting, others have passed it and written
+// their part.  The caller reads b again, so it must not take this form where b is x.
 #pragma once
 #include <algorithm>
 #include <mutex>

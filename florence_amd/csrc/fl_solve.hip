@@ -80,7 +80,10 @@ static int pcg(const int32_t *indptr, const int32_t *node_nbr_ptr, const int32_t
         return FL_E_ARG;
     }
     const int32_t *deg = reinterpret_cast<const int32_t *>(hs + 8);
-    const CgpPlan plan = cgp_plan(nnode, deg[2], deg[0], (1 << 30) - deg[1]);
+    CgpPlan plan = cgp_plan(nnode, deg[2], deg[0], (1 << 30) - deg[1]);
+    // the way back below reads b again, and a workgroup that gives up in the last step leaves the
+    // parts of x that others have written
+    if (b == x) plan.nw = 0;
     if (plan.nw) {
         // the whole solve in one launch
         CgpArgs<VT> a = {};

@@ -120,3 +120,24 @@ def test_pcg_zero_right_hand_side(cuda):
     x = ls.Solve(dm, V, free, torch.zeros(K.shape[0], dtype=torch.float64, device=cuda),
                  torch.full((K.shape[0],), 3.0, dtype=torch.float64, device=cuda))
     assert ls.iterations == [0] and torch.all(x == 0)
+
+
+def test_pcg_in_place(cuda):
+    """b and x in one array: a one-launch solve that gave up would have lost b, so the solve
+    takes the launch-per-step form, bitwise (the one-launch form sums in another order)."""
+    import torch
+    from florence_amd import _lib
+    from florence_amd.solver import LinearSolver
+    m, dm, V, K = _setup()
+    free = torch.as_tensor(np.isnan(clamp_and_pull(m).ravel()).astype(np.uint8), device=cuda)
+    b = torch.as_tensor(np.random.default_rng(4).standard_normal(K.shape[0]), device=cuda) * free
+    lib = _lib.load()
+    ls = LinearSolver(rtol=1e-10)
+    try:
+        _lib.check(lib.fl_set_tuning(_lib.FL_TUNE_CG, 1), "fl_set_tuning")
+        ref = ls.Solve(dm, V, free, b, torch.empty_like(b))
+    finally:
+        lib.fl_set_tuning(_lib.FL_TUNE_CG, 0)
+    x = b.clone()
+    ls.Solve(dm, V, free, x, x)
+    assert torch.equal(x, ref)
