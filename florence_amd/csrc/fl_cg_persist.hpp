@@ -26,15 +26,14 @@
 // has read it, and that is complete before A(k+1), the last meeting before z(k+2) is
 // looked for.  All of it at agent scope: the XCDs' L2s do not see each other's writes.
 //
-// All workgroups must be resident at once: at most one per CU is launched, one such
-// solve per device runs at a time in a process (persistent_lock), and every wait is bounded: a
+// All workgroups must be resident at once: at most one per CU is launched, a process's
+// launches on one device follow one another (PersistentTurn), and every wait is bounded: a
 // workgroup that waits longer than wait_ticks raises the abort flag and returns, the others
 // follow, and the caller solves with the launch-per-step form.  x is undefined then: where
 // the wait that runs out is one for the last meeting, others have passed it and written
 // their part.  The caller reads b again, so it must not take this form where b is x.
 #pragma once
 #include <algorithm>
-#include <mutex>
 
 #include "fl_common.hpp"
 
@@ -474,9 +473,12 @@ static int cgp_launch_k(const CgpPlan &p, const CgpArgs<VT> &a, hipStream_t st) 
     if (p.lds > 64 * 1024)
         FL_HIP_CHECK(hipFuncSetAttribute((const void *)cg_persistent_kernel<VT, K>,
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds));
+    PersistentTurn turn;
+    const int rc = turn.enter(st);
+    if (rc) return rc;
     cg_persistent_kernel<VT, K><<<(unsigned)p.nw, CGP_T, p.lds, st>>>(a);
     FL_LAUNCH_CHECK();
-    return 0;
+    return turn.leave(st);
 }
 
 template <typename VT>

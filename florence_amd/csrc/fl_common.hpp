@@ -54,9 +54,15 @@ struct Carve {
 enum TuneKey { TUNE_STIFF_MINW = 1, TUNE_STIFF_VARIANT_BASE = 2, TUNE_STIFF_SF = 7, TUNE_GATHER = 8, TUNE_CG = 9, TUNE_KEYS = 10 };
 int tuning_value(int key, int dflt);
 
-// Held from the launch of a kernel whose workgroups wait for each other until it has ended:
-// two of them on one device could each hold part of the CUs and wait for the rest.
-std::mutex &persistent_lock(int device);
+// A kernel whose workgroups wait for each other: two of them on one device could each hold part
+// of the CUs and wait for the rest.  Between enter and leave the device's launches of such
+// kernels are this thread's, and st waits for the one before, on whichever stream it is: they
+// follow one another on the device, and no thread waits on the host for another's solve.
+struct PersistentTurn {
+    std::unique_lock<std::mutex> lock;
+    int enter(hipStream_t st);
+    int leave(hipStream_t st);   // after the launch
+};
 
 // Order of the direct scatter table of hexes of p1^3 nodes: the order in which the
 // factorised stiffness kernel stores an element's entries.  Per element and slice az,

@@ -1058,9 +1058,6 @@ int fl_mg_pcg(const FlMgLevel *levels, int32_t nlevels, int32_t v32, const float
     if (b == x) m.cg.nw = 0;   // the way back below reads b again
     bool aborted = false;
     if (m.cg.nw) {
-        int dev = 0;
-        FL_HIP_CHECK(hipGetDevice(&dev));
-        std::lock_guard<std::mutex> lock(persistent_lock(dev));
         cgp_empty_kernel<<<(CGP_SLOTS + 255) / 256, 256, 0, st>>>(m.slots, CGP_SLOTS);
         const int rc = fcg(m, b, x, rO, rOld, p, q, rtol, maxit, check_every, iterations, rel_residual, &aborted);
         if (rc || !aborted) return rc;

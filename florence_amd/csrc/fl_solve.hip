@@ -17,9 +17,36 @@
 
 namespace fl {
 
-std::mutex &persistent_lock(int device) {
-    static std::mutex m[64];
-    return m[device & 63];
+// a device's last launch that PersistentTurn saw; the event lives as long as the process
+struct PersistentDevice {
+    std::mutex m;
+    hipEvent_t last = nullptr;
+};
+static PersistentDevice &persistent_device(int device) {
+    static PersistentDevice d[64];
+    return d[device & 63];
+}
+
+int PersistentTurn::enter(hipStream_t st) {
+    int dev = 0;
+    FL_HIP_CHECK(hipGetDevice(&dev));
+    PersistentDevice &d = persistent_device(dev);
+    lock = std::unique_lock<std::mutex>(d.m);
+    if (!d.last) {
+        FL_HIP_CHECK(hipEventCreateWithFlags(&d.last, hipEventDisableTiming));
+        return 0;
+    }
+    FL_HIP_CHECK(hipStreamWaitEvent(st, d.last, 0));
+    return 0;
+}
+
+int PersistentTurn::leave(hipStream_t st) {
+    int dev = 0;
+    FL_HIP_CHECK(hipGetDevice(&dev));
+    const hipError_t e = hipEventRecord(persistent_device(dev).last, st);
+    lock.unlock();
+    FL_HIP_CHECK(e);
+    return 0;
 }
 
 template <typename VT>
@@ -105,9 +132,6 @@ static int pcg(const int32_t *indptr, const int32_t *node_nbr_ptr, const int32_t
         a.maxit = maxit;
         a.check_every = check_every;
         a.rtol = rtol;
-        int dev = 0;
-        FL_HIP_CHECK(hipGetDevice(&dev));
-        std::lock_guard<std::mutex> lock(persistent_lock(dev));
         cgp_empty_kernel<<<(CGP_SLOTS + 255) / 256, 256, 0, st>>>(slots, CGP_SLOTS);
         const int rc = cgp_launch(plan, a, st);
         if (rc) return rc;
