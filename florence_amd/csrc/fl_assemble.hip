@@ -870,14 +870,17 @@ static size_t gather_lds_bytes(GatherForm f, int deg, int npe) {
     return (size_t)(gather_eb(f) * npe + deg + 1) / 2 * 8 + (size_t)deg * 9 * 8 + 16;
 }
 
-// One past the last class that shares class b's launch, with the greatest degree in *deg:
-// for elements of at most 64 nodes (a wave a node), the classes whose LDS leaves a CU all its
-// 32 waves, or whose nodes are all on the chip at once.  A class of less LDS has no use for a
-// launch of its own then (the gather of 3,072 elements of 10 nodes 28 -> 23 us, 162 of 20 36 ->
-// 21, 48 of 35 59 -> 30, 750 of 35 80 -> 63; in one launch at any size the least class would
-// run at the greatest's occupancy).
-static int gather_classes(const int32_t *bucket_offsets, const int32_t *bucket_degree, int b, int npe, int *deg) {
+// One past the last class that shares class b's launch, with the greatest degree in *deg and,
+// in *merged, whether one of them holds nodes (empty classes are passed over, and a class
+// alone keeps its own form): for elements of at most 64 nodes (a wave a node), the classes whose
+// LDS leaves a CU all its 32 waves, or whose nodes are all on the chip at once.  A class of
+// less LDS has no use for a launch of its own then (the gather of 3,072 elements of 10 nodes
+// 28 -> 23 us, 162 of 20 36 -> 21, 48 of 35 59 -> 30, 750 of 35 80 -> 63; in one launch at any
+// size the least class would run at the greatest's occupancy).
+static int gather_classes(const int32_t *bucket_offsets, const int32_t *bucket_degree, int b, int npe, int *deg,
+                          bool *merged) {
     int next = b + 1;
+    *merged = false;
     if (npe > 64 || tuning_value(TUNE_GATHER, 0) != 0) return next;
     for (; next < FL_GATHER_BUCKETS; ++next) {
         if (bucket_offsets[next + 1] == bucket_offsets[next]) continue;
@@ -885,6 +888,7 @@ static int gather_classes(const int32_t *bucket_offsets, const int32_t *bucket_d
         const size_t lds = gather_lds_bytes(gather_form(1, d, npe), d, npe), cu = 160 * 1024 / (lds ? lds : 1);
         if (cu < 32 && bucket_offsets[next + 1] - bucket_offsets[b] > (int64_t)(256 * cu)) break;
         *deg = d;
+        *merged = true;
     }
     return next;
 }
@@ -1721,11 +1725,12 @@ static int df_assemble(int32_t material, const double *params, const int32_t *el
     }
     for (int b = fuse_interior ? 1 : 0, next; b < FL_GATHER_BUCKETS; b = next) {
         int dg = bucket_degree[b];
-        next = gather_classes(bucket_offsets, bucket_degree, b, npe, &dg);
+        bool merged;
+        next = gather_classes(bucket_offsets, bucket_degree, b, npe, &dg, &merged);
         const int32_t nb = bucket_offsets[next] - bucket_offsets[b];
         if (nb <= 0) continue;
         // several classes: the form of one of more than one element
-        const int fb = next > b + 1 ? 1 : b;
+        const int fb = merged ? 1 : b;
         int rc2 = 0;
         const int32_t *ord = node_order + bucket_offsets[b];
         if (precision == FL_PREC_FP64)

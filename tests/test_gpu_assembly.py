@@ -609,3 +609,48 @@ def test_orphan_node(cuda):
     x = deformed(m2.points, 0.05, seed=4)
     dm, V, T = _check(m2, fs, mat, x, "hex p2 with an orphan point")
     assert np.all(T[-3:] == 0.0)
+
+
+def _kernels_of(fn, path):
+    """The kernels that a call launches: it is captured, and the HIP runtime describes the graph."""
+    import ctypes
+    import re
+    import torch
+    from florence_amd import _lib
+    fn()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        fn()
+    dot = _lib.load().hipGraphDebugDotPrint   # of the runtime that the library is linked to
+    dot.argtypes = [ctypes.c_void_p, ctypes.c_char_p, ctypes.c_uint]
+    assert dot(g.raw_cuda_graph(), str(path).encode(), 1) == 0
+    return re.findall(r"_ZN2fl\d+([a-z0-9_]+_kernel)", path.read_text())
+
+
+@pytest.mark.parametrize("p", [1, 2, 4])
+def test_gather_form_of_separate_elements(cuda, tmp_path, p):
+    """Tets that share no node: every node is in class 0, which has nothing to be merged with
+    and keeps the single-element form; a connected mesh of so few elements is one launch of
+    the general form.  K and T against the oracle."""
+    import torch
+    from florence_amd import Mesh
+    from florence_amd.assembly import DeviceMeshData, assemble_device
+    m = cube_mesh("tet", p, 1, jitter=0.02, seed=p)
+    el, X = np.asarray(m.elements, dtype=np.int64), np.asarray(m.points)
+    apart = Mesh()
+    apart.element_type, apart.points = "tet", X[el.ravel()]
+    apart.elements = np.arange(el.size).reshape(el.shape)
+    apart.InferPolynomialDegree()
+    apart.ChangeType()
+    mat = NeoHookean(3, mu=1.0, lamb=10.0)
+    for mesh, single in ((apart, True), (m, False)):
+        fs = function_space(mesh, p)
+        x = deformed(mesh.points, 0.05, seed=4)
+        if single:
+            _check(mesh, fs, mat, x, "separate tets p{}".format(p))
+        dm = DeviceMeshData(mesh, fs)
+        xd = torch.as_tensor(x, device="cuda")
+        V, T, _ = assemble_device(dm, mat, xd)
+        names = _kernels_of(lambda: assemble_device(dm, mat, xd, V, T), tmp_path / "assembly.dot")
+        assert [k for k in names if "gather" in k] == ["gather_single_kernel" if single else "gather_kernel"]
