@@ -1115,21 +1115,28 @@ static int launch_stiffness_direct(int npe, int G, const double *qp, const void 
         // p = 4: five slices do not fit in LDS; FP64 takes 4 waves (8 spill at the 128 registers
         // that two workgroups leave each: 16^3 3840 against 2613), FP32 8 (4^3 98 against 109,
         // 16^3 within 2 %, and 4 spill where float sums go to double values).
-        // split, a workgroup a slice: where three workgroups an element are fewer than two a CU.
-        // It repeats the loads and tables for every slice and pays where the chip is idle
-        // (together -> split: p = 4, 4^3 458 -> 148, 8^3 577 -> 467; p = 3, 10^3 216 -> 190),
-        // not where it is full (p = 4, 12^3 with 216 elements a colour 1312 -> 1355, 16^3
-        // 2613 -> 2915; p = 3, 17^3 861 -> 884)
+        // A workgroup a slice where three workgroups an element are fewer than two a CU.  It
+        // repeats the loads and tables for every slice and pays where the chip is idle (together ->
+        // a slice each: p = 4, 4^3 458 -> 148, 8^3 577 -> 467; p = 3, 10^3 216 -> 190), not where it is
+        // full (p = 4, 16^3 2613 -> 2915; p = 3, 17^3 861 -> 884).  p = 4 in FP64 has two workgroups
+        // of five slices a CU: launches of one to five and a half a CU are few enough for the last
+        // round to count, and two slices a workgroup even it out (whole assembly by the rule of
+        // p = 3 -> with pairs, us, 6^3 Gauss-Lobatto / 5^3 Gauss points: 9^3 695 -> 663 / 692 -> 651,
+        // 11^3 1200 -> 1070 / 1202 -> 1054, 12^3 1403 -> 1314 / 1448 -> 1315, 14^3 2094 -> 1960 / 2216 ->
+        // 1966, 15^3, colours of 343 to 512 elements, 2432 -> 2358 / 2551 -> 2359; 16^3, 512 elements
+        // a colour, 2772 -> 2836).  In FP32 pairs cost up to 8 % from 12^3 on.
 #define FL_ROWS_CASE(P, QQ, SW, OCC)                                                                                \
     if (npe == P * P * P && G == QQ * QQ * QQ) {                                                                    \
-        const int split = SW > 1 && 3 * n < 2 * 256 ? 1 : 0;                                                     \
-        const int64_t groups = (n + 7) / 8 * 8 * 3 * (split ? P : 1);                                               \
+        const bool f5 = P == 5 && sizeof(CT) == 8;                                                                  \
+        const int64_t wg = 3 * n;                                                                                   \
+        const int ng = SW == 1 ? 1 : (wg < (f5 ? 256 : 512) ? P : (f5 && wg < 1408 ? 3 : 1));                       \
+        const int64_t groups = (n + 7) / 8 * 8 * 3 * ng;                                                            \
         if (groups > (int64_t)INT32_MAX) {                                                                          \
             set_error("too many elements of one colour for one launch");                                            \
             return FL_E_LIMIT;                                                                                      \
         }                                                                                                           \
         stiffness_rows_kernel<P, QQ, SW, OCC, CT, VT><<<(unsigned)groups, SW == 1 ? 64 * P : 64 * SW, 0, st>>>(     \
-            qp, b, n, V, el, elements, indptr, scat, split);                                                        \
+            qp, b, n, V, el, elements, indptr, scat, ng);                                                           \
         FL_LAUNCH_CHECK();                                                                                          \
         continue;                                                                                                   \
     }

@@ -26,13 +26,13 @@ namespace fl {
 
 // SW waves share a slice az.  SW = 1 (WAVE): a workgroup of P1 waves, each with a slice and its
 // own part of LDS to itself, so that no barrier follows the loads.  SW > 1: the waves share
-// out the eta tiles and the column tiles, and the slices follow one another or, with split,
-// go to workgroups of their own (the caller's rule).
+// out the eta tiles and the column tiles, and the slices follow one another in ng workgroups:
+// all of them in one, one in each of P1, or two in each but the last (the caller's rule).
 template <int P1, int Q, int SW, int OCC, typename CT, typename VT>
 __global__ __launch_bounds__(SW == 1 ? 64 * P1 : 64 * SW, OCC) void stiffness_rows_kernel(
     const double *__restrict__ qp, const int32_t *__restrict__ basis, int64_t n, VT *__restrict__ V,
     const int32_t *__restrict__ elist, const int32_t *__restrict__ elements, const int32_t *__restrict__ indptr,
-    const int16_t *__restrict__ scat, int split) {
+    const int16_t *__restrict__ scat, int ng) {
     typedef SfLayout<P1, Q> L;
     typedef Mfma16<CT> MF;
     // output rows of the beta product (and the scatter table's order): the FP64 MFMA's, rows
@@ -63,7 +63,6 @@ __global__ __launch_bounds__(SW == 1 ? 64 * P1 : 64 * SW, OCC) void stiffness_ro
     int16_t *sTg = reinterpret_cast<int16_t *>(&sT2_[0][0][0][0][0]);
     static_assert(sizeof(int16_t) * Q3 <= sizeof(sT2_), "sTg in sT2's space");
 
-    const int ng = split ? P1 : 1;
     const int64_t wid = blockIdx.x;
     const int64_t slot = wid >> 3;
     const int sub = (int)(slot % (3 * ng));
@@ -148,7 +147,8 @@ __global__ __launch_bounds__(SW == 1 ? 64 * P1 : 64 * SW, OCC) void stiffness_ro
     const bool av = arow < PP, ev = ecol < P1 * Q;
     const int arc = av ? arow : 0, ecc = ev ? ecol : 0;
     const int ebz = ecc / Q, eqb = ecc - ebz * Q;   // bz, qb of the column
-    const int z0 = WAVE ? wave : (split ? sub / 3 : 0), z1 = WAVE || split ? z0 + 1 : P1;
+    const int nz = WAVE || ng == P1 ? 1 : (ng == 1 ? P1 : 2);   // a workgroup's slices
+    const int z0 = WAVE ? wave : sub / 3 * nz, z1 = min(z0 + nz, P1);
     for (int az = z0; az < z1; ++az) {
         // the slice's scatter entries: lane's rows (tm, r) of column tile sw + SW v
         TV tv[TW];
@@ -161,7 +161,12 @@ __global__ __launch_bounds__(SW == 1 ? 64 * P1 : 64 * SW, OCC) void stiffness_ro
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             // zeta (VALU): task (mn, qe qb) holds its Q tensor values and sweeps bz
-            for (int t = zid; t < 9 * QQ; t += 64 * SW) {
+            int zt = zid;
+            // one round of tasks: without this the compiler keeps the indices of all three blocks over
+            // the kernel, and Q = 5 spills six registers instead of two (16^3 2890 -> 2780 us; where
+            // there are two rounds, as at Q = 6, or registers to spare it costs 1 to 4 %)
+            if constexpr (F64 && MT > 1 && 9 * QQ <= 64 * SW) asm volatile("" : "+v"(zt));
+            for (int t = zt; t < 9 * QQ; t += 64 * SW) {
                 const int mn = t / QQ, qeb = t - mn * QQ;   // qeb = qb * Q + qe
                 const int m = mn / 3, c = mn - 3 * m;
                 const int qb = qeb / Q, qe = qeb - qb * Q;

@@ -654,3 +654,27 @@ def test_gather_form_of_separate_elements(cuda, tmp_path, p):
         V, T, _ = assemble_device(dm, mat, xd)
         names = _kernels_of(lambda: assemble_device(dm, mat, xd, V, T), tmp_path / "assembly.dot")
         assert [k for k in names if "gather" in k] == ["gather_single_kernel" if single else "gather_kernel"]
+
+
+@pytest.mark.parametrize("points", [5, 6])
+def test_direct_scatter_slice_pairs(cuda, points):
+    """p=4 colours of 64 to 125 elements: both the workgroup a slice and the two slices a
+    workgroup (the last of an element holds one).  FP64 and FP32 blocks against the gather
+    over stored blocks, as above."""
+    import torch
+    from florence_amd.assembly import DeviceMeshData, assemble_device
+    m = cube_mesh("hex", 4, 9, jitter=0.03, seed=9)
+    fs = function_space(m, 4, qtype="lobatto" if points == 6 else "gauss", norder=points)
+    mat = MooneyRivlin(3, mu1=0.5, mu2=0.5, lamb=20.0)
+    x = deformed(m.points, 0.003, seed=10)
+    dm = DeviceMeshData(m, fs)
+    assert dm.ngauss == points ** 3
+    sizes = np.diff(list(dm.colour_offsets)[:dm.ncolour + 1])
+    assert sizes.min() == 64 and sizes.max() == 125
+    for kw in ({}, {"precision": "fp32"}):
+        V, T, st = assemble_device(dm, mat, x, **kw)
+        V, T = V.clone(), T.clone()
+        assert int(st[0].item()) == 0
+        Vg, Tg, _ = assemble_device(dm, mat, x, direct=False, **kw)
+        assert float((V - Vg).abs().max() / Vg.abs().max()) <= 1e-13
+        assert torch.equal(T, Tg)
