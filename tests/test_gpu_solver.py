@@ -141,3 +141,12 @@ def test_pcg_in_place(cuda):
     x = b.clone()
     ls.Solve(dm, V, free, x, x)
     assert torch.equal(x, ref)
+
+
+@pytest.mark.parametrize("element,p,n,csr", [("tet", 2, 12, "fp64"), ("tet", 2, 13, "fp64"), ("tet", 3, 7, "fp64"),
+                                             ("hex", 2, 10, "fp32"), ("hex", 4, 3, "fp64")])
+def test_pcg_in_one_launch_largest_forms(cuda, element, p, n, csr):
+    """The matrices above come to one, two and four blocks per thread in up to 63 KB of LDS.
+    These come to four in 91 KB, and to five, the most there are, in 115, 88, 80 and 65 KB
+    (on 256 CUs); the same checks."""
+    test_pcg_in_one_launch(cuda, element, p, n, csr)
