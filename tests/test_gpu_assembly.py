@@ -678,3 +678,33 @@ def test_direct_scatter_slice_pairs(cuda, points):
         Vg, Tg, _ = assemble_device(dm, mat, x, direct=False, **kw)
         assert float((V - Vg).abs().max() / Vg.abs().max()) <= 1e-13
         assert torch.equal(T, Tg)
+
+
+@pytest.mark.parametrize("p,points,form", [(2, 79, "stiffness_el_kernel"), (2, 80, "stiffness_kernel"),
+                                           (3, 64, "stiffness_el_kernel"), (3, 65, "stiffness_kernel"),
+                                           (4, 46, "stiffness_el_kernel"), (4, 47, "stiffness_kernel")])
+def test_dense_form_by_points(cuda, tmp_path, p, points, form):
+    """The most points of which the element form of the dense contraction takes 10, 20 and 35
+    nodes, and one more, which the pair form takes: its default FP64 shapes of the
+    16-, 32- and 48-node classes, which no tabulated rule reaches any more (variant 0 of the
+    test of the tile variants is the element form for these node counts).  The rule
+    is any: positive weights at points inside the element.  Against the oracle."""
+    import torch
+    from florence_amd.assembly import DeviceMeshData, assemble_device
+    from florence_amd.function_space import FunctionSpace
+    from florence_amd.quadrature import QuadratureRule
+    rng = np.random.default_rng(points)
+    q = QuadratureRule(mesh_type="tet", evaluate=False)
+    bary = rng.dirichlet(np.ones(4), points)
+    q.points = bary @ np.array([[-1.0, -1, -1], [1, -1, -1], [-1, 1, -1], [-1, -1, 1]])
+    q.weights = (0.5 + rng.random(points)) * (4.0 / 3.0) / points
+    m = cube_mesh("tet", p, 1, jitter=0.05, seed=31)
+    fs = FunctionSpace(m, q, p=p)
+    mat = MooneyRivlin(3, mu1=0.5, mu2=0.5, lamb=20.0)
+    x = deformed(m.points, 0.05, seed=32)
+    _check(m, fs, mat, x, "tet p{} G={}".format(p, points))
+    dm = DeviceMeshData(m, fs)
+    xd = torch.as_tensor(x, device="cuda")
+    V, T, _ = assemble_device(dm, mat, xd)
+    names = _kernels_of(lambda: assemble_device(dm, mat, xd, V, T), tmp_path / "assembly.dot")
+    assert [k for k in names if k.startswith("stiffness")] == [form]
