@@ -395,7 +395,7 @@ class WarmStartMLP(object):
         if self._buf.get("n", 0) < n:
             f32 = dict(dtype=torch.float32, device=self.device)
             self._buf = {"n": n, "H1": torch.empty((n, H), **f32), "H2": torch.empty((n, H), **f32),
-                         "Y": torch.empty((n, OP), **f32), "F": torch.empty((n, IP), **f32)}
+                         "Y": torch.empty((n, OP), **f32)}
         return self._buf
 
     def forward(self, F, n):
