@@ -886,7 +886,7 @@ static int gather_classes(const int32_t *bucket_offsets, const int32_t *bucket_d
         if (bucket_offsets[next + 1] == bucket_offsets[next]) continue;
         const int d = *deg > bucket_degree[next] ? *deg : bucket_degree[next];
         const size_t lds = gather_lds_bytes(gather_form(1, d, npe), d, npe), cu = 160 * 1024 / (lds ? lds : 1);
-        if (cu < 32 && bucket_offsets[next + 1] - bucket_offsets[b] > (int64_t)(256 * cu)) break;
+        if (cu < 32 && bucket_offsets[next + 1] - bucket_offsets[b] > (int64_t)(device_cus() * cu)) break;
         *deg = d;
         *merged = true;
     }
@@ -1105,6 +1105,7 @@ static int launch_stiffness_direct(int npe, int G, const double *qp, const void 
                                    const int32_t *indptr, int ncolour, const int32_t *offsets,
                                    const int32_t *elems, const int16_t *scat, VT *V, hipStream_t st) {
     const int32_t *b = static_cast<const int32_t *>(basis);
+    const int cus = device_cus();
     for (int c = 0; c < ncolour; ++c) {
         const int64_t n = offsets[c + 1] - offsets[c];
         if (n <= 0) continue;
@@ -1129,7 +1130,7 @@ static int launch_stiffness_direct(int npe, int G, const double *qp, const void 
     if (npe == P * P * P && G == QQ * QQ * QQ) {                                                                    \
         const bool f5 = P == 5 && sizeof(CT) == 8;                                                                  \
         const int64_t wg = 3 * n;                                                                                   \
-        const int ng = SW == 1 ? 1 : (wg < (f5 ? 256 : 512) ? P : (f5 && wg < 1408 ? 3 : 1));                       \
+        const int ng = SW == 1 ? 1 : (wg < (f5 ? cus : 2 * cus) ? P : (f5 && 2 * wg < 11 * cus ? 3 : 1));           \
         const int64_t groups = (n + 7) / 8 * 8 * 3 * ng;                                                            \
         if (groups > (int64_t)INT32_MAX) {                                                                          \
             set_error("too many elements of one colour for one launch");                                            \
@@ -1200,7 +1201,8 @@ static int launch_points_t(const MatParams &mp, const double *points, const int3
         // three more waves share the tractions' sums where all workgroups are on the chip at
         // once (four a CU: 375 groups of 35 nodes 23 us against 29 with one wave); beyond that
         // they only take the place of other workgroups (2,187 groups 63 against 56)
-        qp_traction_kernel<TANGENT, GEN><<<(unsigned)groups, groups <= 1024 ? 256 : 64, points_lds(G, npe), st>>>(
+        const int threads = groups <= 4 * device_cus() ? 256 : 64;
+        qp_traction_kernel<TANGENT, GEN><<<(unsigned)groups, threads, points_lds(G, npe), st>>>(
             mp, points, elements, Eulerx, Jm, JmT, NP, w, G, nelem, npe, update, TANGENT ? qp : nullptr, status,
             elem_mat, mat_table, te);
     } else {

@@ -446,10 +446,8 @@ __global__ __launch_bounds__(CGP_T) void cg_persistent_kernel(CgpArgs<VT> A) {
 constexpr int CGP_PER_WG = 740;
 static CgpPlan cgp_plan(int64_t nnode, int64_t total, int maxdeg, int mindeg) {
     CgpPlan p;
-    int dev = 0, cus = 0;
-    if (total <= 0 || mindeg < 1 || tuning_value(TUNE_CG, 0) == 1 || hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        return p;
+    const int cus = device_cus();
+    if (total <= 0 || mindeg < 1 || cus <= 0 || tuning_value(TUNE_CG, 0) == 1) return p;
     const int most_wg = std::min(cus, CGP_MAXW), per_1 = CGP_T - maxdeg;
     const int per_wg = per_1 > CGP_T / 2 && total <= (int64_t)most_wg * per_1 ? per_1 : CGP_PER_WG;
     const int nw = (int)std::min<int64_t>(most_wg, (total + per_wg - 1) / per_wg);

@@ -54,6 +54,10 @@ struct Carve {
 enum TuneKey { TUNE_STIFF_MINW = 1, TUNE_STIFF_VARIANT_BASE = 2, TUNE_STIFF_SF = 7, TUNE_GATHER = 8, TUNE_CG = 9, TUNE_KEYS = 10 };
 int tuning_value(int key, int dflt);
 
+// CUs of the current device (a partition has fewer than the chip's 256), by which the dispatch
+// rules count their workgroups; 0 where they cannot be had.
+int device_cus();
+
 // A kernel whose workgroups wait for each other: two of them on one device could each hold part
 // of the CUs and wait for the rest.  Between enter and leave the device's launches of such
 // kernels are this thread's, and st waits for the one before, on whichever stream it is: they

@@ -8,6 +8,7 @@
 // A = M K M + (I - M) with M = diag(free), which keeps the CSR untouched; every
 // iterate vanishes on fixed dofs.  All reductions are two-pass with a fixed order,
 // so a solve is bitwise reproducible.
+#include <atomic>
 #include <cmath>
 #include <vector>
 
@@ -16,6 +17,18 @@
 #include "fl_solve_kernels.hpp"
 
 namespace fl {
+
+int device_cus() {
+    static std::atomic<int> known[64];
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 0;
+    std::atomic<int> &k = known[dev & 63];
+    n = k.load(std::memory_order_relaxed);
+    if (n) return n;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 0;
+    k.store(n, std::memory_order_relaxed);
+    return n;
+}
 
 // a device's last launch that PersistentTurn saw; the event lives as long as the process
 struct PersistentDevice {
