@@ -4,8 +4,9 @@
 // ComputeSparsityPattern.pyx:44-90, ComputeSparsityPattern.h:22-62): for node a the
 // sorted unique set of nodes sharing an element with it; its three rows 3a+i list the
 // columns 3b+k of every neighbour b in ascending order.  The reference builds this per
-// node with std::sort/std::unique on the host; here one workgroup per node gathers the
-// candidate nodes of its incident elements into LDS, bitonic-sorts them and compacts.
+// node with std::sort/std::unique on the host; here one wave per node (a workgroup where a
+// node has more than 1024 candidates) gathers the candidate nodes of its incident
+// elements into LDS, bitonic-sorts them and compacts.
 #include <cstdarg>
 #include <climits>
 #include <algorithm>
@@ -477,7 +478,7 @@ static unsigned group_grid(int64_t nnode) { return (unsigned)std::min<int64_t>((
 // their scan per class, and a stable scatter.
 constexpr int PL_CHUNK = 1024, PL_C = FL_GATHER_BUCKETS;
 // scratch (int32, zeroed): [0] 2^30 - smallest count, [1, 7) largest count per class, [7, 13)
-// nodes per class, [13] largest count above every class; from 16: [chunk][class]
+// nodes per class, [13] INT32_MAX - the first node above every class; from 16: [chunk][class]
 constexpr int PL_HEAD = 16;
 __device__ __forceinline__ int plan_class(int d, int dmin) {
     if (d == dmin) return 0;
@@ -500,18 +501,19 @@ __global__ __launch_bounds__(256) void plan_min_kernel(const int32_t *__restrict
 template <bool SCATTER>
 __global__ __launch_bounds__(256) void plan_chunk_kernel(const int32_t *__restrict__ ptr, int64_t nnode,
                                                          int32_t *__restrict__ w, int32_t *__restrict__ order) {
-    __shared__ int32_t cnt[4][PL_C], base[PL_C], deg[PL_C + 1];
+    __shared__ int32_t cnt[4][PL_C], base[PL_C], deg[PL_C];
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
     const int dmin = (1 << 30) - w[0];
     int32_t *hist = w + PL_HEAD + PL_C * (int64_t)blockIdx.x;
     if (t < PL_C) base[t] = SCATTER ? hist[t] : 0;
-    if (t < PL_C + 1) deg[t] = 0;
+    if (t < PL_C) deg[t] = 0;
     __syncthreads();
     for (int r = 0; r < PL_CHUNK / 256; ++r) {
         const int64_t a = (int64_t)blockIdx.x * PL_CHUNK + 256 * r + t;
         const int d = a < nnode ? ptr[a + 1] - ptr[a] : 0;
         const int c = a < nnode ? plan_class(d, dmin) : -1;
-        if (!SCATTER && c >= 0 && d > deg[c]) atomicMax(&deg[c], d);
+        if (!SCATTER && c == PL_C) atomicMax(w + 13, INT32_MAX - (int32_t)a);
+        if (!SCATTER && c >= 0 && c < PL_C && d > deg[c]) atomicMax(&deg[c], d);
         int before = 0;
 #pragma unroll
         for (int k = 0; k < PL_C; ++k) {
@@ -533,7 +535,6 @@ __global__ __launch_bounds__(256) void plan_chunk_kernel(const int32_t *__restri
             hist[t] = base[t];
             if (deg[t]) atomicMax(w + 1 + t, deg[t]);
         }
-        if (t == PL_C && deg[t]) atomicMax(w + 13, deg[t]);
     }
 }
 
@@ -796,7 +797,12 @@ int fl_pattern_gather_plan(const int32_t *node_nbr_ptr, int64_t nnode, int32_t *
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     FL_HIP_CHECK(e);
     if (h[13] > 0) {
-        set_error("fl_pattern_gather_plan: a node has %d neighbours (limit %d)", h[13], 64 << (PL_C - 1));
+        const int64_t a = INT32_MAX - h[13];
+        int32_t p[2] = {0, 0};
+        FL_HIP_CHECK(hipMemcpyAsync(p, node_nbr_ptr + a, sizeof(p), hipMemcpyDeviceToHost, st));
+        FL_HIP_CHECK(hipStreamSynchronize(st));
+        set_error("fl_pattern_gather_plan: node %lld has %d neighbours (limit %d)", (long long)a, p[1] - p[0],
+                  64 << (PL_C - 1));
         return FL_E_LIMIT;
     }
     bucket_offsets[0] = 0;

@@ -80,3 +80,16 @@ def test_gather_plan_limit(cuda):
     el, nnode = _star(700, 4)     # node 0 has 2101 neighbours
     with pytest.raises(_lib.FlorenceAMDError, match="limit 2048"):
         _device_pattern(el, nnode)
+
+
+def test_gather_plan_limit_names_the_node(cuda):
+    """The error names the first node above the limit and its count.  Two centres of 700 tets
+    each: nodes 5 and 3000, of 2101 neighbours."""
+    a, na = _star(700, 4)
+    b, nb = _star(700, 4)
+    el = np.concatenate([a, b + na])
+    ids = np.arange(na + nb)
+    ids[[0, 5]] = [5, 0]
+    ids[[na, 3000]] = [3000, na]
+    with pytest.raises(_lib.FlorenceAMDError, match=r"node 5 has 2101 neighbours \(limit 2048\)"):
+        _device_pattern(ids[el].astype(np.int32), na + nb)
