@@ -95,7 +95,7 @@ __device__ __forceinline__ double ws_corrected(double a, double b, float y, cons
 // bounds it is latency: at 11664 rows the three products are 0.6 GFLOP and 14 MB of
 // activations.  As three 64 x 64-tile products through memory (one load per element,
 // converted in the inner loop) they took 52 us; this kernel takes 9.5 us at 8192 rows and,
-// with the inputs and outputs below fused in, 11.4 us at 11664 (56 us in five launches).
+// with the inputs and outputs below fused in, 10.2 us at 11664 (56 us in five launches).
 // PREDICT: the inputs are formed from the nodes' states and the outputs added to
 // the extrapolation in the same launch (no activation reaches memory).
 template <bool PREDICT>

@@ -301,9 +301,9 @@ struct SfLines {
 // Bound by VALU issue and LDS together
 // (p = 4, 6^3 points: 1004 VALU and 163 LDS instructions a wave, half the cycles each); a
 // task an output, which reads both factors of every product from LDS, and a workgroup an
-// element at every p were LDS-bound, and idle at small p.  Residual pass before -> now: p = 4,
-// 20^3 elements 229 -> 125 us, p = 2, 25^3 89 -> 44, p = 1, 20^3 37 -> 29; the point phase of
-// the assembly: 352 -> 230, 182 -> 68, 77 -> 26.  A thread takes record point g, not tensor
+// element at every p were LDS-bound, and idle at small p.  Residual pass before -> now (us): p = 4,
+// 20^3 elements 185 -> 107 with 6^3 points, 148 -> 85 with 5^3, p = 2, 22^3 60 -> 35, p = 1, 30^3 95 ->
+// 31; the point phase of the assembly, p = 4, 20^3: 352 -> 230.  A thread takes record point g, not tensor
 // point g: its wave's 54 record stores are then contiguous (p = 4, 20^3 284 -> 230).  Two points a thread, for half of P's reads,
 // do not pay (134, and 617 for the tangent, whose registers then spill).
 template <int P1, int Q, bool TANGENT, bool GEN>

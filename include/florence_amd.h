@@ -460,7 +460,8 @@ int32_t fl_stiffness_variant_count(int32_t np_class);
 /* key 9: block-Jacobi CG (fl_pcg, fl_mg_pcg's coarsest level) -- 1: one launch per step's
  * part for every matrix; 2: the one-launch form gives up its first wait, and the solve
  * falls back to the other (the results are those of 1).  Default: one launch per solve
- * where the matrix fits the chip's registers. */
+ * where the matrix fits the chip's registers and b is not x.  Such launches of one process
+ * follow one another on a device, on whichever streams they are. */
 #define FL_TUNE_CG 9
 int fl_set_tuning(int32_t key, int32_t value);
 int fl_profile_read(int32_t *kinds, double *phase_ms, int32_t max_calls, int32_t max_phases);
