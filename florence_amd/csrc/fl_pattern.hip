@@ -5,7 +5,7 @@
 // sorted unique set of nodes sharing an element with it; its three rows 3a+i list the
 // columns 3b+k of every neighbour b in ascending order.  The reference builds this per
 // node with std::sort/std::unique on the host; here one wave per node (a workgroup where a
-// node has more than 1024 candidates) gathers the candidate nodes of its incident
+// node has many candidates) gathers the candidate nodes of its incident
 // elements into LDS, bitonic-sorts them and compacts.
 #include <cstdarg>
 #include <climits>
@@ -233,13 +233,24 @@ __device__ int gather_sort_unique(const int32_t *__restrict__ elements, int32_t 
     return flag_sum[NB_T - 1];
 }
 
-// Nodes of at most NW_MAX candidates: one wave per node, its candidates sorted in the
+// Nodes of at most rule.wave_max candidates: one wave per node, its candidates sorted in the
 // wave's own 4 KB of LDS without a workgroup barrier (a wave's LDS accesses are in order;
 // the fences only keep the compiler's).  The workgroup form below, for the nodes above
 // that, sorted every list before: its 33 KB of LDS and two dozen barriers for lists of
 // mostly under 64 candidates took 292 + 170 us on 24k tet p=2 nodes; this form
 // takes 28 + 33.
 constexpr int NW_MAX = 1024;
+
+struct ListRule {
+    int wave_max;   // candidates of a node that a wave takes, at most NW_MAX
+    int per;        // nodes a workgroup of the other form looks through at a time, at most NB_T
+};
+// A mesh of few nodes waits for its longest list, which a lone wave sorts more slowly than a
+// workgroup, and leaves the chip room for a workgroup a node: both passes of p = 4 tets, 793
+// nodes 224 -> 184 us, 5,681 nodes 243 -> 208; p = 4 hexes, 729 nodes 230 -> 186, 4,913 249 -> 225
+// (lists above 256 only: 204, 222, 207, 234).  From there on workgroups wait for each other: p = 3
+// hexes, 6,859 nodes 189 -> 194, p = 4 hexes, 15,625 nodes 262 -> 404.
+static ListRule list_rule(int64_t nnode) { return nnode <= 6144 ? ListRule{128, 1} : ListRule{NW_MAX, NB_T}; }
 
 __device__ __forceinline__ void wave_fence() {
     __builtin_amdgcn_wave_barrier();
@@ -267,7 +278,7 @@ constexpr int32_t FILL_BAD = INT32_MIN;   // in indptr[3 nnode]: lists inconsist
 template <bool FILL>
 __global__ __launch_bounds__(256) void wave_neighbours_kernel(
     const int32_t *__restrict__ elements, int32_t npe, const int32_t *__restrict__ node_elem_ptr,
-    const int32_t *__restrict__ node_elem, int64_t nnode, int64_t *__restrict__ nbr_count,
+    const int32_t *__restrict__ node_elem, int64_t nnode, ListRule rule, int64_t *__restrict__ nbr_count,
     const int32_t *__restrict__ node_nbr_ptr, int32_t *__restrict__ node_nbrs, int32_t *__restrict__ indptr,
     int32_t *__restrict__ indices) {
     __shared__ int32_t sc[4][NW_MAX];
@@ -277,7 +288,7 @@ __global__ __launch_bounds__(256) void wave_neighbours_kernel(
     if (a >= nnode) return;
     const int32_t b0 = node_elem_ptr[a];
     const int64_t nc = (int64_t)(node_elem_ptr[a + 1] - b0) * npe;
-    if (nc > NW_MAX) return;
+    if (nc > rule.wave_max) return;
     const int ncand = (int)nc;
     int S = 64;
     while (S < ncand) S <<= 1;
@@ -328,21 +339,21 @@ __global__ __launch_bounds__(256) void wave_neighbours_kernel(
     }
 }
 
-// The nodes of more than NW_MAX candidates, one workgroup per node: a grid of fixed size
-// looks through the nodes 256 at a time and takes up the large ones.
+// The nodes of more candidates than a wave takes, one workgroup per node: a grid of fixed
+// size looks through the nodes rule.per at a time and takes up the large ones.
 template <bool FILL>
 __global__ __launch_bounds__(NB_T) void group_neighbours_kernel(
     const int32_t *__restrict__ elements, int32_t npe, const int32_t *__restrict__ node_elem_ptr,
-    const int32_t *__restrict__ node_elem, int64_t nnode, int64_t *__restrict__ nbr_count,
+    const int32_t *__restrict__ node_elem, int64_t nnode, ListRule rule, int64_t *__restrict__ nbr_count,
     int32_t *__restrict__ overflow, const int32_t *__restrict__ node_nbr_ptr,
     int32_t *__restrict__ node_nbrs, int32_t *__restrict__ indptr, int32_t *__restrict__ indices) {
     __shared__ int32_t cand[NB_MAX];
     __shared__ int32_t flag_sum[NB_T];
     __shared__ unsigned long long large[NB_T / 64];
     const int t = threadIdx.x;
-    for (int64_t base = (int64_t)blockIdx.x * NB_T; base < nnode; base += (int64_t)gridDim.x * NB_T) {
-        const bool mine = base + t < nnode &&
-                          (int64_t)(node_elem_ptr[base + t + 1] - node_elem_ptr[base + t]) * npe > NW_MAX;
+    for (int64_t base = (int64_t)blockIdx.x * rule.per; base < nnode; base += (int64_t)gridDim.x * rule.per) {
+        const bool mine = t < rule.per && base + t < nnode &&
+                          (int64_t)(node_elem_ptr[base + t + 1] - node_elem_ptr[base + t]) * npe > rule.wave_max;
         const unsigned long long m = __ballot(mine);
         if ((t & 63) == 0) large[t >> 6] = m;
         __syncthreads();
@@ -468,7 +479,9 @@ __global__ void scatter_table_kernel(const int32_t *__restrict__ elements, int64
     table[t] = ok ? (int16_t)(add ? lo - 32768 : lo) : (int16_t)0;
 }
 
-static unsigned group_grid(int64_t nnode) { return (unsigned)std::min<int64_t>((nnode + NB_T - 1) / NB_T, 1024); }
+static unsigned group_grid(int64_t nnode, int per) {
+    return (unsigned)(per == 1 ? nnode : std::min<int64_t>((nnode + per - 1) / per, 1024));
+}
 
 // ------------------------------------------------------------------- gather plan
 // Node classes by neighbour count: class 0 the smallest count (in meshes with
@@ -621,11 +634,11 @@ int fl_pattern_graph(const int32_t *elements, int64_t nelem, int32_t npe, int64_
                                                                                         node_elem_ptr);
     FL_LAUNCH_CHECK();
     FL_HIP_CHECK(hipMemsetAsync(nbrc, 0, sizeof(int64_t) * (nnode + 1), st));
+    const ListRule rule = list_rule(nnode);
     wave_neighbours_kernel<false><<<(unsigned)((nnode + 3) / 4), 256, 0, st>>>(
-        elements, npe, node_elem_ptr, node_elem, nnode, nbrc, nullptr, nullptr, nullptr, nullptr);
-    group_neighbours_kernel<false><<<group_grid(nnode), NB_T, 0, st>>>(elements, npe, node_elem_ptr, node_elem, nnode,
-                                                                      nbrc, flags + 1, nullptr, nullptr,
-                                                                      nullptr, nullptr);
+        elements, npe, node_elem_ptr, node_elem, nnode, rule, nbrc, nullptr, nullptr, nullptr, nullptr);
+    group_neighbours_kernel<false><<<group_grid(nnode, rule.per), NB_T, 0, st>>>(
+        elements, npe, node_elem_ptr, node_elem, nnode, rule, nbrc, flags + 1, nullptr, nullptr, nullptr, nullptr);
     FL_LAUNCH_CHECK();
     rc = exclusive_scan_i64(nbrc, nnode + 1, scratch, sc, st);
     if (rc) return rc;
@@ -665,11 +678,11 @@ int fl_pattern_fill(const int32_t *elements, int64_t nelem, int32_t npe, int64_t
     // the last entry of indptr carries the kernels' flag to the host: FILL_BAD, or the total
     int32_t *last = indptr + 3 * nnode;
     FL_HIP_CHECK(hipMemsetAsync(last, 0, sizeof(int32_t), st));
+    const ListRule rule = list_rule(nnode);
     wave_neighbours_kernel<true><<<(unsigned)((nnode + 3) / 4), 256, 0, st>>>(
-        elements, npe, node_elem_ptr, node_elem, nnode, nullptr, node_nbr_ptr, node_nbrs, indptr, indices);
-    group_neighbours_kernel<true><<<group_grid(nnode), NB_T, 0, st>>>(elements, npe, node_elem_ptr, node_elem, nnode,
-                                                                     nullptr, last, node_nbr_ptr, node_nbrs,
-                                                                     indptr, indices);
+        elements, npe, node_elem_ptr, node_elem, nnode, rule, nullptr, node_nbr_ptr, node_nbrs, indptr, indices);
+    group_neighbours_kernel<true><<<group_grid(nnode, rule.per), NB_T, 0, st>>>(
+        elements, npe, node_elem_ptr, node_elem, nnode, rule, nullptr, last, node_nbr_ptr, node_nbrs, indptr, indices);
     FL_LAUNCH_CHECK();
     int32_t h = 0;
     FL_HIP_CHECK(hipMemcpyAsync(&h, last, sizeof(int32_t), hipMemcpyDeviceToHost, st));

@@ -93,3 +93,15 @@ def test_gather_plan_limit_names_the_node(cuda):
     ids[[na, 3000]] = [3000, na]
     with pytest.raises(_lib.FlorenceAMDError, match=r"node 5 has 2101 neighbours \(limit 2048\)"):
         _device_pattern(ids[el].astype(np.int32), na + nb)
+
+
+@pytest.mark.parametrize("star", [(16, 4), (64, 10), (65, 4), (256, 4), (257, 4), (29, 35)])
+def test_pattern_of_many_nodes(cuda, monkeypatch, star):
+    """The stars above beside a strip that makes the mesh one of many nodes, where one wave
+    takes lists of up to 1024 candidates (of few nodes: 128, the rest a workgroup a node)."""
+    el, n = _star(*star)
+    more, m = _strip(6200 // (star[1] - 1), star[1], 1)
+    both = np.concatenate([el, more + n]).astype(np.int32)
+    assert n + m > 6144
+    monkeypatch.setitem(globals(), "_star", lambda *a: (both, n + m))
+    test_pattern_equals_oracle(cuda, ("star",) + star)
